@@ -7,7 +7,8 @@ A case is a dict of plain values:
   ``ctx_lo .. ctx_hi`` tokens; ``prompts`` sequences bring ``new_lo .. new_hi`` new tokens each
   over ``pre_lo .. pre_hi`` tokens that are cached already. A step of decode rows alone takes
   the decode kernel, any other step the variable-length one, as the engine's context says.
-* ``kind`` "compress": one layer's compression step of ``topk`` sequences out of a batch.
+* ``kind`` "compress": one layer's compression step of ``topk`` sequences out of a batch, whose
+  windows' tokens were stored since the step before (a step leaves the kept rows in their place).
 * ``kind`` "norm_rope": q/k RMSNorm + RoPE + cache store of ``tokens`` tokens.
 
 ``hq``/``hk`` are the query and KV heads of one GPU (head_dim 128, blocks of 256 tokens), ``kv``
@@ -225,8 +226,11 @@ def _run_attention(s):
 
 def _prepare_compress(case, gen, host):
     lens, chosen = _compress_lengths(case)
-    # only the chosen sequences' blocks are touched: the others own none here
+    # only the chosen sequences' blocks are touched: the others own one each here
     table, pool = _tables([n if i in set(chosen) else 1 for i, n in enumerate(lens)], host)
+    pos = [(lens[i] // BLOCK - WINDOW) * BLOCK + torch.arange(WINDOW * BLOCK) for i in chosen]
+    slots = torch.cat([table[i, p // BLOCK].long() * BLOCK + p % BLOCK
+                       for i, p in zip(chosen, pos)]).to(torch.int32)
     hq, hk, m = case["hq"], case["hk"], len(chosen)
     sets, cand = (1 if case["agg"] == "all" else hk), WINDOW * BLOCK - 1
     k_cache, v_cache = _caches(case, pool, gen)
@@ -234,6 +238,9 @@ def _prepare_compress(case, gen, host):
     need = compress_utils.select_workspace_bytes(m, hq, hk, WINDOW, BLOCK)
     return dict(
         kind="compress", agg=case["agg"], k_scale=K_SCALE if case["kv"] == "fp8" else 1.0,
+        v_scale=V_SCALE if case["kv"] == "fp8" else 1.0, slots=slots.cuda(),
+        k=_randn(gen, slots.numel(), hk, D, dtype=_dtype(case)),
+        v=_randn(gen, slots.numel(), hk, D, dtype=_dtype(case)),
         q=_randn(gen, len(lens), hq, D, dtype=_dtype(case), scale=2.0), k_cache=k_cache,
         v_cache=v_cache, table=table.cuda(), base=base, lens=base.clone(),
         chosen=torch.tensor(chosen, dtype=torch.int32).cuda(),
@@ -244,6 +251,8 @@ def _prepare_compress(case, gen, host):
 
 
 def _run_compress(s):
+    nkv.store_kvcache(s["k"], s["v"], s["k_cache"], s["v_cache"], s["slots"], s["k_scale"],
+                      s["v_scale"])
     keep, importance = compress_utils.compress_step(
         s["q"], s["k_cache"], s["v_cache"], s["table"], s["base"], s["lens"], s["chosen"],
         WINDOW, KEEP, SCALE, s["agg"], importance=s["importance"], keep_idx=s["keep"],
@@ -312,10 +321,12 @@ def work(case):
     if case["kind"] == "compress":
         lens, chosen = _compress_lengths(case)
         m, tails = len(chosen), sum(lens[i] % BLOCK for i in chosen)
-        # the window's K, the kept V, the tails; kept and tail rows written; q
+        # the windows' new rows read and stored; the windows' K, the kept V and the tails read;
+        # kept and tail rows written; q
+        stored = 2 * m * WINDOW * BLOCK
         read = m * (WINDOW * BLOCK + KEEP) + 2 * tails
         written = 2 * (m * KEEP + tails)
-        return dict(bytes=(read + written) * row + m * hq * D * 2,
+        return dict(bytes=stored * (hk * D * 2 + row) + (read + written) * row + m * hq * D * 2,
                     flops=2 * m * hq * D * WINDOW * BLOCK)
     n = case["tokens"]
     heads = hq + 2 * hk
@@ -343,19 +354,21 @@ def _values(cache, scale, fp8):
     return cache.double() * (scale if fp8 else 1.0)
 
 
+def _stored(s, kc, vc, hk, fp8):
+    """The new K/V rows in their slots of the caches."""
+    rows = s["slots"].long()
+    for cache, x, scale in ((kc, s["k"], K_SCALE), (vc, s["v"], V_SCALE)):
+        if fp8:
+            x = (x.float() * (1.0 / scale)).clamp(-448, 448).to(torch.float8_e4m3fn)
+        _whole(cache).view(-1, hk * D)[rows] = _whole(x).view(-1, hk * D)
+
+
 def _exact_attention(case, s):
     fp8 = case["kv"] == "fp8"
     hq, hk = case["hq"], case["hk"]
     g = hq // hk
     kc, vc = s["layer"].k_cache, s["layer"].v_cache
-    rows = s["slots"].long()
-    if fp8:
-        for cache, x, scale in ((kc, s["k"], K_SCALE), (vc, s["v"], V_SCALE)):
-            codes = (x.float() * (1.0 / scale)).clamp(-448, 448).to(torch.float8_e4m3fn)
-            _whole(cache).view(-1, hk * D)[rows] = codes.view(torch.uint8).view(-1, hk * D)
-    else:
-        kc.view(-1, hk * D)[rows] = s["k"].view(-1, hk * D)
-        vc.view(-1, hk * D)[rows] = s["v"].view(-1, hk * D)
+    _stored(s, kc, vc, hk, fp8)
     out = torch.empty(sum(s["new"]), hq, D, dtype=torch.float64, device="cuda")
     at = 0
     for i, (lq, lk) in enumerate(zip(s["new"], s["keys"])):
@@ -384,6 +397,7 @@ def _exact_compress(case, s):
     hq, hk = case["hq"], case["hk"]
     g, w = hq // hk, WINDOW * BLOCK
     lens, chosen = _compress_lengths(case)
+    _stored(s, s["k_cache"], s["v_cache"], hk, fp8)
     importance = torch.empty(len(chosen), hk, w - 1, dtype=torch.float64, device="cuda")
     for j, i in enumerate(chosen):
         full = lens[i] // BLOCK
