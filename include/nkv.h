@@ -322,6 +322,37 @@ int nkv_prefill_varlen_f16(const void* q, int64_t q_row_stride,
                            int32_t block_size, int64_t n_rows, float scale,
                            void* out, int64_t out_row_stride, void* stream);
 
+/* Element type of K/V (q and out are bf16 over an fp8 pool, K/V's type otherwise). */
+#define NKV_KV_BF16 0
+#define NKV_KV_F16 1
+#define NKV_KV_FP8 2
+
+/* Varlen causal prefill with the keys split over the chip: the arguments of
+ * nkv_prefill_varlen (kv_type NKV_KV_BF16), nkv_prefill_varlen_f16 (NKV_KV_F16) or, paged only,
+ * nkv_prefill_varlen_fp8 (NKV_KV_FP8: row strides in codes, n_rows = blocks * block_size,
+ * the scales used), the same results up to the order of the sums over keys. Every
+ * workgroup takes an equal share of all (sequence, tile, key step) work, whatever the mix of
+ * lengths, and a second kernel merges the tiles whose keys were shared out; the plain entry
+ * points give each tile's keys to one workgroup. The workspace (16-byte aligned,
+ * nkv_prefill_split_workspace_bytes; independent of the lengths) holds the parts; calls that
+ * overlap need one each. */
+size_t nkv_prefill_split_workspace_bytes(int32_t n_q_heads, int32_t n_kv_heads,
+                                         int32_t head_dim, int32_t kv_type);
+/* The same bytes where the split launch is expected to be the faster one for n_seqs sequences
+ * with total_q rows of q and the given longest lengths, else 0 (take a plain entry point). */
+size_t nkv_prefill_split_plan(int32_t n_seqs, int64_t total_q, int32_t max_seqlen_q,
+                              int32_t max_seqlen_k, int32_t n_q_heads, int32_t n_kv_heads,
+                              int32_t head_dim, int32_t kv_type);
+int nkv_prefill_varlen_split(int32_t kv_type, const void* q, int64_t q_row_stride,
+                             const void* k_cache, const void* v_cache, int64_t k_row_stride,
+                             int64_t v_row_stride, const int32_t* cu_seqlens_q,
+                             const int32_t* cu_seqlens_k, const int32_t* block_tables,
+                             int64_t bt_row_stride, int32_t max_blocks_per_seq, int32_t n_seqs,
+                             int32_t max_seqlen_q, int32_t n_q_heads, int32_t n_kv_heads,
+                             int32_t head_dim, int32_t block_size, int64_t n_rows, float scale,
+                             float k_scale, float v_scale, void* out, int64_t out_row_stride,
+                             void* workspace, size_t workspace_bytes, void* stream);
+
 /* Aggregation of key importance over query heads (compression scoring). */
 #define NKV_AGG_ALL 0   /* sum over all Hq heads -> one kept set per sequence
                            (nanokvllm/layers/CompressMethod.py:41-42) */

@@ -20,6 +20,9 @@ LIB_PATH = os.path.join(PKG_DIR, "libnkv_amd.so")
 DEBUG_LIB_PATH = os.path.join(PKG_DIR, "libnkv_amd_debug.so")
 
 NKV_OK = 0
+NKV_KV_BF16 = 0
+NKV_KV_F16 = 1
+NKV_KV_FP8 = 2
 NKV_AGG_ALL = 0
 NKV_AGG_GROUP = 1
 NKV_DECODE_NOALLOC_MAX_BYTES = 64 << 20  # include/nkv.h
@@ -72,6 +75,11 @@ SIGNATURES = {
     "nkv_prefill_varlen_fp8": (C.c_int, [_p, _i64, _p, _p, _p, _p, _p, _i64, _i32, _i32, _i32,
                                          _i32, _i32, _i32, _i32, _i64, _f32, _f32, _f32, _p,
                                          _i64, _p]),
+    "nkv_prefill_split_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32]),
+    "nkv_prefill_split_plan": (_sz, [_i32, _i64, _i32, _i32, _i32, _i32, _i32, _i32]),
+    "nkv_prefill_varlen_split": (C.c_int, [_i32, _p, _i64, _p, _p, _i64, _i64, _p, _p, _p, _i64,
+                                           _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i64, _f32,
+                                           _f32, _f32, _p, _i64, _p, _sz, _p]),
     "nkv_compress_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32]),
     "nkv_compress_score": (C.c_int, [_p, _i64, _p, _p, _i64, _i32, _p, _p, _i32, _i32, _i32, _i32,
                                      _i32, _i32, _i64, _f32, _i32, _p, _p, _sz, _p]),

@@ -26,6 +26,9 @@ void clear_error();
 // Checks the launch just issued on the current thread.
 int check_launch(const char* what);
 
+// Compute units of the current device (cached per device; 256 when it cannot be queried).
+int device_cus();
+
 // Input checks of the debug build (-DNKV_DEBUG, libnkv_amd_debug.so): NKV_DBG(cond, bit)
 // ORs an NKV_DEBUG_* bit into this source file's device word when cond holds, and each
 // source file registers a reader of its word with nkv_debug_flags. Without NKV_DEBUG the
@@ -139,6 +142,17 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// Inclusive prefix sum over the wave's lanes.
+__device__ __forceinline__ int wave_incl_scan(int v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(v, o, 64);
+    if (lane >= o) v += y;
+  }
+  return v;
+}
+
 // max(a, b, c) as one v_maximum3_f32 (no operand canonicalisation; NaN-propagating)
 __device__ __forceinline__ float fmax3(float a, float b, float c) {
   return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
@@ -165,6 +179,42 @@ __device__ __forceinline__ float col_sum4(float v) {
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// N consecutive floats of a partial row (N = D / 64 output dims per lane).
+template <int N>
+__device__ __forceinline__ void load_dims(const float* p, float (&v)[N]) {
+  if constexpr (N == 1) {
+    v[0] = *p;
+  } else if constexpr (N == 2) {
+    const float2 t = *reinterpret_cast<const float2*>(p);
+    v[0] = t.x;
+    v[1] = t.y;
+  } else {
+    static_assert(N == 4, "1, 2 or 4 dims per lane");
+    const float4 t = *reinterpret_cast<const float4*>(p);
+    v[0] = t.x;
+    v[1] = t.y;
+    v[2] = t.z;
+    v[3] = t.w;
+  }
+}
+// N output dims of one lane as bf16 or fp16 (2, 4 or 8 bytes).
+template <bool H16>
+__device__ __forceinline__ uint32_t out_pk(float lo, float hi) {
+  if constexpr (H16) return cvt_pk16<true>(lo, hi);
+  else return pack_bf16x2(lo, hi);
+}
+template <int N, bool H16>
+__device__ __forceinline__ void store_dims(bf16_t* op, const float (&o)[N], float scale) {
+  if constexpr (N == 1) {
+    *reinterpret_cast<uint16_t*>(op) = (uint16_t)(out_pk<H16>(o[0] * scale, 0.f) & 0xffffu);
+  } else if constexpr (N == 2) {
+    *reinterpret_cast<uint32_t*>(op) = out_pk<H16>(o[0] * scale, o[1] * scale);
+  } else {
+    *reinterpret_cast<uint2*>(op) =
+        uint2{out_pk<H16>(o[0] * scale, o[1] * scale), out_pk<H16>(o[2] * scale, o[3] * scale)};
+  }
+}
 
 constexpr float kLog2e = 1.4426950408889634f;
 

@@ -3,6 +3,8 @@
 
 #include <string.h>
 
+#include <atomic>
+
 namespace nkv {
 
 static thread_local char g_last_error[512] = "";
@@ -23,6 +25,21 @@ int check_launch(const char* what) {
     return NKV_ELAUNCH;
   }
   return NKV_OK;
+}
+
+int device_cus() {
+  // threads that race here compute and store the same value
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  int n = cached[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        n <= 0)
+      n = 256;
+    cached[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
 }
 
 // Readers of the debug words of every source file (debug build), registered while the

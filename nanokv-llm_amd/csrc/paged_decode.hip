@@ -91,16 +91,6 @@ static inline int32_t decode_min_chunks(int32_t max_blocks, int32_t block_size) 
   return (int32_t)(c > kMinChunks ? c : kMinChunks);
 }
 
-__device__ __forceinline__ int wave_incl_scan(int v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(v, o, 64);
-    if (lane >= o) v += y;
-  }
-  return v;
-}
-
 // Cursor over sequences in batches of 64 (one per lane): in the chunk stream
 // of one KV head, sequence s owns chunks [g_s, g_s + nc_s).
 struct SeqCursor {
@@ -462,42 +452,6 @@ void paged_decode_split_kernel(
   }
 }
 
-// N consecutive floats of a partial row (N = D / 64 output dims per lane).
-template <int N>
-__device__ __forceinline__ void load_dims(const float* p, float (&v)[N]) {
-  if constexpr (N == 1) {
-    v[0] = *p;
-  } else if constexpr (N == 2) {
-    const float2 t = *reinterpret_cast<const float2*>(p);
-    v[0] = t.x;
-    v[1] = t.y;
-  } else {
-    static_assert(N == 4, "1, 2 or 4 dims per lane");
-    const float4 t = *reinterpret_cast<const float4*>(p);
-    v[0] = t.x;
-    v[1] = t.y;
-    v[2] = t.z;
-    v[3] = t.w;
-  }
-}
-// N output dims of one lane as bf16 or fp16 (2, 4 or 8 bytes).
-template <bool H16>
-__device__ __forceinline__ uint32_t out_pk(float lo, float hi) {
-  if constexpr (H16) return cvt_pk16<true>(lo, hi);
-  else return pack_bf16x2(lo, hi);
-}
-template <int N, bool H16>
-__device__ __forceinline__ void store_dims(bf16_t* op, const float (&o)[N], float scale) {
-  if constexpr (N == 1) {
-    *reinterpret_cast<uint16_t*>(op) = (uint16_t)(out_pk<H16>(o[0] * scale, 0.f) & 0xffffu);
-  } else if constexpr (N == 2) {
-    *reinterpret_cast<uint32_t*>(op) = out_pk<H16>(o[0] * scale, o[1] * scale);
-  } else {
-    *reinterpret_cast<uint2*>(op) =
-        uint2{out_pk<H16>(o[0] * scale, o[1] * scale), out_pk<H16>(o[2] * scale, o[3] * scale)};
-  }
-}
-
 // Merge the partials of one (sequence, query head): O = sum_s 2^(m_s-M) O_s /
 // sum_s 2^(m_s-M) l_s. One wave per pair; lane l owns output dims N*l .. N*l+N-1.
 template <int D, bool H16 = false>
@@ -609,22 +563,6 @@ static int decode_check(const void* q, const void* k_cache, const void* v_cache,
   NKV_REQUIRE(aligned16(q) && aligned16(k_cache) && aligned16(v_cache), NKV_EINVAL,
               "paged_decode: q/k_cache/v_cache must be 16-byte aligned");
   return NKV_OK;
-}
-
-// Compute units of the current device (cached per device; 256 when it cannot be queried).
-static int device_cus() {
-  // threads that race here compute and store the same value
-  static std::atomic<int> cached[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  int n = cached[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        n <= 0)
-      n = 256;
-    cached[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
 }
 
 // Persistent grid: as many one-wave workgroups as are resident at once, at most

@@ -192,11 +192,28 @@ def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     return out
 
 
+_SPLIT_MIN_KEYS = 512  # the plan never splits shorter contexts: not asked for them
+
+
+def varlen_prefill_workspace(q: torch.Tensor, k: torch.Tensor, n_seqs: int, max_seqlen_q: int,
+                             max_seqlen_k: int) -> torch.Tensor | None:
+    """The workspace for splitting varlen_prefill's keys where that is the faster way (a few
+    query tiles, or a long context among short ones: the longest sequence would otherwise hold
+    the call up), else None. Sized by the chip, not by the lengths."""
+    t = _lib.NKV_KV_FP8 if k.dtype == torch.float8_e4m3fn else \
+        _lib.NKV_KV_F16 if k.dtype == torch.float16 else _lib.NKV_KV_BF16
+    nbytes = _lib.lib().nkv_prefill_split_plan(n_seqs, q.size(0), int(max_seqlen_q),
+                                               int(max_seqlen_k), q.size(1), k.size(-2),
+                                               q.size(2), t)
+    return torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+
+
 def varlen_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                    cu_seqlens_q: torch.Tensor, cu_seqlens_k: torch.Tensor, max_seqlen_q: int,
                    scale: float, block_tables: torch.Tensor | None = None,
                    out: torch.Tensor | None = None, max_seqlen_k: int | None = None,
-                   k_scale: float = 1.0, v_scale: float = 1.0) -> torch.Tensor:
+                   k_scale: float = 1.0, v_scale: float = 1.0,
+                   workspace: torch.Tensor | None = None) -> torch.Tensor:
     """Varlen causal (bottom-right) attention: q [sum Lq, Hq, D] -> [sum Lq, Hq, D].
 
     With ``block_tables`` k/v are the paged caches [NB, B, Hk, D]; without,
@@ -204,6 +221,9 @@ def varlen_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     contiguous, v a view of the qkv projection). Same math as
     flash_attn_varlen_func(..., causal=True, block_table) at attention.py:96-102.
     q, k, v and the output are bf16 or fp16 (one dtype); an fp8 pool takes bf16 q.
+    With a ``workspace`` (varlen_prefill_workspace) the keys are split over the chip, equal
+    shares of all the work to every workgroup; without, each query tile's keys stay with one
+    workgroup and nothing but the output is allocated.
     """
     N, Hq, D = q.shape
     _lib.require_device(q.device, k=k, v=v, cu_seqlens_q=cu_seqlens_q, cu_seqlens_k=cu_seqlens_k,
@@ -220,34 +240,24 @@ def varlen_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         _lib.need(out.shape == q.shape and out.dtype == q.dtype and out.stride(-1) == 1
                   and out.stride(1) == D, "varlen_prefill: out must be shaped like q, in q's "
                   "dtype, rows of contiguous heads")
-    if block_tables is not None and k.dtype == torch.float8_e4m3fn:
-        # fp8 pool: the kernel widens the codes as it stages them (no bf16 copy)
-        NB, B, Hk, Dk = k.shape
-        _lib.need(not f16, "varlen_prefill: an fp8 pool is read with bf16 q")
-        _lib.need(v.shape == k.shape and k.is_contiguous() and v.is_contiguous(),
-                  "varlen_prefill: fp8 caches must be contiguous, v shaped like k")
-        _lib.need(block_tables.dtype == torch.int32 and block_tables.stride(1) == 1,
-                  "varlen_prefill: block_tables must be int32 rows")
-        assert Dk == D
-        if out is None:
-            out = torch.empty(N, Hq, D, dtype=_BF16, device=q.device)
-        rc = _lib.lib().nkv_prefill_varlen_fp8(
-            q.data_ptr(), q.stride(0), k.data_ptr(), v.data_ptr(), cu_seqlens_q.data_ptr(),
-            cu_seqlens_k.data_ptr(), block_tables.data_ptr(), block_tables.stride(0),
-            block_tables.size(1), n_seqs, int(max_seqlen_q), Hq, Hk, D, B, NB, float(scale),
-            float(k_scale), float(v_scale), out.data_ptr(), out.stride(0), _lib.stream_of(q))
-        _lib.check(rc, "varlen_prefill_fp8")
-        return out
+    fp8 = block_tables is not None and k.dtype == torch.float8_e4m3fn
     if block_tables is not None:
         NB, B, Hk, Dk = k.shape
-        assert k.is_contiguous() and v.is_contiguous() and v.shape == k.shape
-        _lib.need(k.dtype == q.dtype, "varlen_prefill: paged caches must have q's dtype "
-                  "(or be fp8)")
+        if fp8:  # the kernel widens the codes as it stages them (no bf16 copy)
+            _lib.need(not f16, "varlen_prefill: an fp8 pool is read with bf16 q")
+            _lib.need(v.shape == k.shape and k.is_contiguous() and v.is_contiguous(),
+                      "varlen_prefill: fp8 caches must be contiguous, v shaped like k")
+            _lib.need(block_tables.dtype == torch.int32 and block_tables.stride(1) == 1,
+                      "varlen_prefill: block_tables must be int32 rows")
+        else:
+            assert k.is_contiguous() and v.is_contiguous() and v.shape == k.shape
+            _lib.need(k.dtype == q.dtype, "varlen_prefill: paged caches must have q's dtype "
+                      "(or be fp8)")
+            assert block_tables.dtype == torch.int32 and block_tables.stride(1) == 1
         k_row_stride = v_row_stride = Hk * Dk
         n_rows = NB * B
         bt_ptr, bt_stride = block_tables.data_ptr(), block_tables.stride(0)
         max_blocks = block_tables.size(1)
-        assert block_tables.dtype == torch.int32 and block_tables.stride(1) == 1
     else:
         _, Hk, Dk = k.shape
         assert v.shape == k.shape
@@ -260,11 +270,34 @@ def varlen_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     assert Dk == D
     if out is None:
         out = torch.empty(N, Hq, D, dtype=q.dtype, device=q.device)
-    fn = _lib.lib().nkv_prefill_varlen_f16 if f16 else _lib.lib().nkv_prefill_varlen
+    lib = _lib.lib()
+    max_q = int(max_seqlen_q)
+    kv_type = _lib.NKV_KV_FP8 if fp8 else _lib.NKV_KV_F16 if f16 else _lib.NKV_KV_BF16
+    if workspace is not None:
+        _lib.require_device(q.device, workspace=workspace)
+        _lib.need(workspace.dtype == torch.uint8 and workspace.is_contiguous(),
+                  "varlen_prefill: workspace must be contiguous uint8")
+        rc = lib.nkv_prefill_varlen_split(
+            kv_type, q.data_ptr(), q.stride(0), k.data_ptr(), v.data_ptr(), k_row_stride,
+            v_row_stride, cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), bt_ptr, bt_stride,
+            max_blocks, n_seqs, max_q, Hq, Hk, D, B, n_rows, float(scale),
+            float(k_scale) if fp8 else 1.0, float(v_scale) if fp8 else 1.0, out.data_ptr(),
+            out.stride(0), workspace.data_ptr(), workspace.numel(), _lib.stream_of(q))
+        _lib.check(rc, "varlen_prefill_split")
+        return out
+    if fp8:
+        rc = lib.nkv_prefill_varlen_fp8(
+            q.data_ptr(), q.stride(0), k.data_ptr(), v.data_ptr(), cu_seqlens_q.data_ptr(),
+            cu_seqlens_k.data_ptr(), bt_ptr, bt_stride, max_blocks, n_seqs, max_q, Hq, Hk, D, B,
+            NB, float(scale), float(k_scale), float(v_scale), out.data_ptr(), out.stride(0),
+            _lib.stream_of(q))
+        _lib.check(rc, "varlen_prefill_fp8")
+        return out
+    fn = lib.nkv_prefill_varlen_f16 if f16 else lib.nkv_prefill_varlen
     rc = fn(
         q.data_ptr(), q.stride(0), k.data_ptr(), v.data_ptr(), k_row_stride, v_row_stride,
         cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), bt_ptr, bt_stride, max_blocks, n_seqs,
-        int(max_seqlen_q), Hq, Hk, D, B, n_rows, float(scale), out.data_ptr(), out.stride(0),
+        max_q, Hq, Hk, D, B, n_rows, float(scale), out.data_ptr(), out.stride(0),
         _lib.stream_of(q))
     _lib.check(rc, "varlen_prefill")
     return out
@@ -371,11 +404,16 @@ class Attention(nn.Module):
 
         if not context.use_decode_kernel:
             if context.block_tables is not None:  # K/V read back from the paged cache
+                workspace = None
+                if context.max_seqlen_k > _SPLIT_MIN_KEYS:
+                    workspace = varlen_prefill_workspace(
+                        q, k_cache, context.cu_seqlens_q.numel() - 1, context.max_seqlen_q,
+                        context.max_seqlen_k)
                 return varlen_prefill(q, k_cache, v_cache, context.cu_seqlens_q,
                                       context.cu_seqlens_k, context.max_seqlen_q, self.scale,
                                       block_tables=context.block_tables,
                                       max_seqlen_k=context.max_seqlen_k, k_scale=self.k_scale,
-                                      v_scale=self.v_scale)
+                                      v_scale=self.v_scale, workspace=workspace)
             return varlen_prefill(q, k, v, context.cu_seqlens_q, context.cu_seqlens_k,
                                   context.max_seqlen_q, self.scale)
         o = paged_decode(q, k_cache, v_cache, context.context_lens, context.block_tables,

@@ -1,0 +1,161 @@
+"""Variable-length attention with the keys split over the chip (nkv_prefill_varlen_split)
+against the fp32 oracle: every form the entry point takes, at lengths around the edges of
+tiles, key steps and ranges, and the launch rule's choice through Attention.forward."""
+import importlib
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from oracle.attention_ref import varlen_prefill_ref
+
+L = importlib.import_module("nanokv-llm_amd._lib")
+TOL = 2e-2  # the repository's bar for 16-bit outputs of N(0, 1) values
+
+# (new tokens, keys) per sequence
+MIXES = {
+    # decode rows, empty sequences, rows that see no key, one chunk on a prefix
+    "mixed": [(1, 900), (0, 0), (1, 1), (0, 70), (49, 333), (1, 1500), (17, 9), (1, 64)],
+    # one row whose keys every range shares
+    "one_row": [(1, 2999)],
+    # tiles of 48 queries at G = 4: one short of, at and one past a tile and a key step
+    "edges": [(47, 63), (48, 64), (49, 65), (96, 128), (97, 1281)],
+    # a sequence per range and more than one batch of 64 sequences
+    "many": [(1 + i % 3, 30 * (i % 7) + 3) for i in range(130)],
+    # one chunk on a long prefix
+    "chunk": [(130, 2311)],
+}
+
+
+def _inputs(dev, mix, Hq, Hk, D, kind, B, paged, seed):
+    g = torch.Generator().manual_seed(seed)
+    dt = torch.float16 if kind == "fp16" else torch.bfloat16
+    lq, lk = [a for a, _ in mix], [b for _, b in mix]
+    cs = lambda x: torch.tensor([0] + x).cumsum(0).to(torch.int32)  # noqa: E731
+    q = torch.randn(sum(lq), Hq, D, generator=g).to(dt)
+    if not paged:  # V a strided view, as of a qkv projection
+        k = torch.randn(sum(lk), Hk, D, generator=g).to(dt)
+        v = torch.randn(sum(lk), 3 * Hk, D, generator=g).to(dt)[:, Hk:2 * Hk]
+        return q, k, v, cs(lq), cs(lk), None
+    need = [-(-n // B) for n in lk]
+    ids = torch.randperm(sum(need) + 3, generator=g).to(torch.int32)
+    bt = torch.full((len(mix), max(need)), -1, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        bt[i, :n] = ids[at:at + n]
+        at += n
+    kv = torch.randn(2, sum(need) + 3, B, Hk, D, generator=g)
+    kv = (kv * 16).to(torch.float8_e4m3fn) if kind == "fp8" else kv.to(dt)
+    return q, kv[0], kv[1], cs(lq), cs(lk), bt
+
+
+def _split(dev, q, k, v, cu_q, cu_k, bt, kind, scale):
+    N, Hq, D = q.shape
+    t = {"bf16": L.NKV_KV_BF16, "fp16": L.NKV_KV_F16, "fp8": L.NKV_KV_FP8}[kind]
+    Hk = k.size(-2)
+    n_rows = k.size(0) * (k.size(1) if bt is not None else 1)
+    ks, vs = (k.stride(0), v.stride(0)) if bt is None else (Hk * D, Hk * D)
+    s = 1 / 16 if kind == "fp8" else 1.0
+    d = [x.to(dev) if x is not None else None for x in (q, k, cu_q, cu_k, bt)]
+    # a strided V stays strided on the device
+    vd = v.to(dev) if v.is_contiguous() else \
+        torch.empty_strided(v.shape, v.stride(), dtype=v.dtype, device=dev).copy_(v)
+    nbytes = L.lib().nkv_prefill_split_workspace_bytes(Hq, Hk, D, t)
+    ws = torch.full((nbytes,), 0xff, dtype=torch.uint8, device=dev)  # NaN where nothing is written
+    out = torch.full((N, Hq, D), float("nan"), dtype=q.dtype, device=dev)
+    max_q = int((cu_q[1:] - cu_q[:-1]).max())
+    L.check(L.lib().nkv_prefill_varlen_split(
+        t, d[0].data_ptr(), q.stride(0), d[1].data_ptr(), vd.data_ptr(), ks, vs,
+        d[2].data_ptr(), d[3].data_ptr(), d[4].data_ptr() if bt is not None else None,
+        bt.stride(0) if bt is not None else 0, bt.size(1) if bt is not None else 0,
+        cu_q.numel() - 1, max_q, Hq, Hk, D, k.size(1) if bt is not None else 0, n_rows, scale,
+        s, s, out.data_ptr(), out.stride(0), ws.data_ptr(), ws.numel(), L.stream_of(d[0])),
+        "prefill_varlen_split")
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mix,Hq,Hk,D,kind,B,paged", [
+    ("mixed", 32, 8, 128, "bf16", 256, True),
+    ("mixed", 20, 4, 128, "fp16", 16, True),    # a group that leaves spare rows; 4 blocks a step
+    ("mixed", 16, 2, 128, "fp8", 64, True),
+    ("mixed", 16, 8, 128, "bf16", 0, False),
+    ("mixed", 8, 4, 64, "bf16", 256, True),
+    ("mixed", 8, 2, 256, "fp16", 64, True),
+    ("mixed", 16, 4, 64, "fp8", 64, True),
+    ("mixed", 4, 2, 256, "fp8", 256, True),
+    ("mixed", 64, 1, 128, "bf16", 256, True),   # a group of 64: three queries a tile
+    ("one_row", 32, 8, 128, "bf16", 256, True),
+    ("one_row", 5, 1, 128, "fp8", 256, True),   # every range one part
+    ("edges", 32, 8, 128, "bf16", 64, True),
+    ("edges", 32, 8, 128, "fp16", 0, False),
+    ("many", 8, 4, 128, "bf16", 16, True),
+    ("many", 8, 2, 128, "fp8", 64, True),
+    ("chunk", 32, 8, 128, "bf16", 256, True),
+    ("chunk", 8, 1, 64, "fp16", 0, False),
+])
+def test_split_matches_the_oracle(dev, mix, Hq, Hk, D, kind, B, paged):
+    print(mix, Hq, Hk, D, kind, B, paged, flush=True)
+    q, k, v, cu_q, cu_k, bt = _inputs(dev, MIXES[mix], Hq, Hk, D, kind, B, paged, seed=5)
+    out = _split(dev, q, k, v, cu_q, cu_k, bt, kind, D ** -0.5)
+    s = 1 / 16 if kind == "fp8" else 1.0
+    ref = varlen_prefill_ref(q.float(), k.float() * s, v.float() * s, cu_q, cu_k, D ** -0.5,
+                             block_tables=bt)
+    assert (out.float().cpu() - ref).abs().max().item() <= TOL
+
+
+@pytest.mark.gpu
+def test_attention_takes_a_long_prefix_to_the_split_launch(nkv, dev):
+    """Attention.forward against the plain launch: two orders of the same sums, each weight
+    and output rounded to bf16 (2^-8 relative, |out| < 1 here); then captured in a graph and
+    replayed over other queries, with eager work between the replays."""
+    mix = [(130, 9000), (1, 400)]
+    q, k, v, cu_q, cu_k, bt = (x.to(dev) for x in
+                               _inputs(dev, mix, 32, 8, 128, "bf16", 256, True, seed=6))
+    assert L.lib().nkv_prefill_split_plan(2, 131, 130, 9000, 32, 8, 128, L.NKV_KV_BF16) > 0
+    layer = nkv.Attention(32, 128, 128 ** -0.5, 8, SimpleNamespace(kv_compress_enabled=False), 1)
+    layer.k_cache, layer.v_cache = k, v
+    nkv.set_context(False, cu_q, cu_k, 130, 9000, None, None, bt)
+    run = lambda: layer(q, None, None, 0, kv_stored=True)  # noqa: E731
+    plain = lambda: nkv.varlen_prefill(q, k, v, cu_q, cu_k, 130, 128 ** -0.5,  # noqa: E731
+                                       block_tables=bt)
+    assert (run().float() - plain().float()).abs().max().item() <= 2 ** -8
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        run()
+    stream.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = run()
+    for scale in (1.0, -0.5, 2.0):
+        q.mul_(scale)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, run())
+    nkv.reset_context()
+
+
+def test_split_plan_and_arguments_on_the_host():
+    """The rule, and what the entry point refuses, without a GPU."""
+    lib = L.lib()
+    plan = lambda *a: lib.nkv_prefill_split_plan(*a)  # noqa: E731
+    full = lib.nkv_prefill_split_workspace_bytes(32, 8, 128, L.NKV_KV_BF16)
+    assert plan(1, 512, 512, 12800, 32, 8, 128, L.NKV_KV_BF16) == full > 0
+    assert plan(50, 1072, 512, 5700, 32, 8, 128, L.NKV_KV_BF16) == full
+    # tiles that fill the chip, short contexts, prompts of many tiles, nothing known
+    assert plan(16, 32768, 2048, 9000, 32, 8, 128, L.NKV_KV_BF16) == 0
+    assert plan(3, 120, 40, 300, 32, 8, 128, L.NKV_KV_BF16) == 0
+    assert plan(1, 20000, 20000, 30000, 32, 8, 128, L.NKV_KV_BF16) == 0
+    assert plan(1, 512, 512, 0, 32, 8, 128, L.NKV_KV_BF16) == 0
+    assert plan(0, 0, 0, 0, 32, 8, 128, L.NKV_KV_BF16) == 0
+    assert plan(1, 512, 512, 12800, 30, 8, 128, L.NKV_KV_BF16) == 0
+
+    def call(kv_type=L.NKV_KV_BF16, ws=1 << 12, nbytes=full, bt=1 << 12):
+        return lib.nkv_prefill_varlen_split(
+            kv_type, 1 << 12, 32 * 128, 1 << 12, 1 << 12, 8 * 128, 8 * 128, 1 << 12, 1 << 12, bt,
+            4, 4, 1, 16, 32, 8, 128, 256, 4 * 256, 1.0, 1.0, 1.0, 1 << 12, 32 * 128, ws, nbytes,
+            None)
+    assert call(kv_type=3) == -1
+    assert call(ws=None) == -3 and call(ws=(1 << 12) + 8) == -3 and call(nbytes=full - 1) == -3
+    assert call(kv_type=L.NKV_KV_FP8, bt=None) == -1  # fp8 rows are paged
