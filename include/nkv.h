@@ -332,11 +332,12 @@ int nkv_prefill_varlen_f16(const void* q, int64_t q_row_stride,
  * nkv_prefill_varlen_fp8 (NKV_KV_FP8: row strides in codes, n_rows = blocks * block_size,
  * the scales used), the same results up to the order of the sums over keys. Every
  * workgroup takes an equal share of all (sequence, tile, key step) work, whatever the mix of
- * lengths, and a second kernel merges the tiles whose keys were shared out; the plain entry
+ * lengths, sequences that bring one token (paged) are streamed as nkv_paged_decode does, and a
+ * second kernel merges the tiles and rows whose keys were shared out; the plain entry
  * points give each tile's keys to one workgroup. The workspace (16-byte aligned,
  * nkv_prefill_split_workspace_bytes; independent of the lengths) holds the parts; calls that
  * overlap need one each. */
-size_t nkv_prefill_split_workspace_bytes(int32_t n_q_heads, int32_t n_kv_heads,
+size_t nkv_prefill_split_workspace_bytes(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads,
                                          int32_t head_dim, int32_t kv_type);
 /* The same bytes where the split launch is expected to be the faster one for n_seqs sequences
  * with total_q rows of q and the given longest lengths, else 0 (take a plain entry point). */

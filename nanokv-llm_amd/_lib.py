@@ -75,7 +75,7 @@ SIGNATURES = {
     "nkv_prefill_varlen_fp8": (C.c_int, [_p, _i64, _p, _p, _p, _p, _p, _i64, _i32, _i32, _i32,
                                          _i32, _i32, _i32, _i32, _i64, _f32, _f32, _f32, _p,
                                          _i64, _p]),
-    "nkv_prefill_split_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32]),
+    "nkv_prefill_split_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32]),
     "nkv_prefill_split_plan": (_sz, [_i32, _i64, _i32, _i32, _i32, _i32, _i32, _i32]),
     "nkv_prefill_varlen_split": (C.c_int, [_i32, _p, _i64, _p, _p, _i64, _i64, _p, _p, _p, _i64,
                                            _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i64, _f32,

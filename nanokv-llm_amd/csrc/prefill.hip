@@ -38,7 +38,11 @@
 //    while this step computes, then widened to bf16 (exact) and written to the
 //    same swizzled LDS rows, so the MFMA part is the bf16 kernel's. The K scale
 //    is folded into the softmax scale, the V scale into the final 1/l.
-#include "nkv_common.h"
+//  * Split launch (nkv_prefill_varlen_split): where few tiles or one long context would leave
+//    the chip idle, the resident workgroups take equal ranges of all (tile, key step) work and a
+//    second kernel merges the cut tiles; decode rows (one new token) are streamed by waves of
+//    workgroups of their own, as the decode kernel does.
+#include "decode_stream.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -47,7 +51,6 @@ namespace nkv {
 
 constexpr int kStep = 64;                 // keys per step
 constexpr int kStages = 2;                // LDS ring depth (steps)
-constexpr int kBufferFlags = 0x00020000;  // raw buffer descriptor word 3 for gfx950
 constexpr bool prefill_dim_ok(int D) { return D == 64 || D == 128 || D == 256; }
 // 16-row groups per wave: three at head_dim 128 (each K and V^T read from LDS serves three
 // MFMAs; bit-identical to two, at par to 2% faster), two at 64 and in the fp8 instance (whose
@@ -71,8 +74,6 @@ __device__ __forceinline__ int chunk_swz(int r) {
 }
 constexpr float kLazy = 8.f;              // log2 headroom before the running max is raised
 
-typedef short i16x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
 typedef __attribute__((address_space(3))) u32x4_t lds_u32x4_t;
 typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
 
@@ -103,9 +104,13 @@ __device__ __forceinline__ void load_to_lds(i32x4_t desc, uint32_t lds_addr, uin
 // What the split launch adds to the plain one's arguments.
 struct SplitArgs {
   int32_t n_seqs;
-  int32_t min_range;  // shortest range, in cost units
-  i32x4_t* desc;      // one per workgroup: {parts, first row of q, queries, 0}
-  float* part;        // two tiles of partial rows per workgroup
+  int32_t min_range;   // shortest range, in cost units
+  i32x4_t* desc;       // one per workgroup: {parts, first row of q, queries, KV head}
+  float* part;         // two tiles of partial rows per workgroup
+  int32_t ncg;         // the decode rows' column groups, their shortest range in chunks,
+  int32_t min_chunks;  // descriptors and partial rows (decode_stream.h)
+  i32x4v_t* row_desc;
+  float* row_part;
 };
 constexpr int kMinRange = 20;  // cost units (four key steps of a full tile)
 constexpr int kSnap = 2;  // a range never cuts a unit within this many steps of its ends
@@ -126,23 +131,38 @@ __device__ __forceinline__ int tile_steps(int Lq, int Lk, int qt, int t) {
   return last >= 0 ? last / kStep + 1 : 1;
 }
 
+// The decode rows among prompts (sequences that bring one new token; HP > 0, the KV heads a
+// wave reads at once) are no units of the stream below: waves of workgroups of their own
+// stream them as the decode kernel does, bound by the K/V bytes, beside the workgroups that
+// the prompts' tiles keep at the matrix cores. A 192-row tile for one row ran at 5.2 TB/s of
+// K/V (a 256-byte piece of each row and 64 keys in flight a workgroup; decode_stream: 6.5).
+// Cost of a 16-key chunk of one head, in quarters of a tile step's units: fewer workgroups than
+// their share of the time alone would give them (5 and 3), since the memory serves the rows
+// at its full rate from half the chip's waves while the others compute. 48 rows with two
+// 512-token chunks, at 1, 2, 3, 4, 6: 116, 117, 126, 129, 160 us; 80 rows of 4k - 8k with one:
+// 333, 319, 316, 361; 60 fp8 rows with two: 88, 111, 119, 125.
+constexpr int row_cost(bool F8) { return F8 ? 1 : 2; }
+
 // The ranges of the split launch. The units of a KV head (sequence, tile) stand in one
 // stream, a unit as long as its cost; range w is [w*C, (w+1)*C), with a cut that falls near
 // a unit's end moved to that end. Every workgroup finds its own range from cu_seqlens.
 struct SplitCursor {
   int seq, tile, q0, Lq, kb0, Lk;  // the current unit
   int u0;                          // its position in the stream
-  int s_lo;                        // first key step of it that belongs to the range
-  int C, T, x_end;                 // range length, stream length, the range's end
+  int C, T, x, x_end;              // range length, stream length, the range's begin and end
+  int group;                       // this workgroup's index among those of the tiles
+  int row_groups;                  // workgroups of the decode rows: the first of the grid
 };
 
-template <int D, bool F8>
+// false: nothing to do, or (row_groups > blockIdx.x) the decode rows.
+template <int D, bool F8, bool ROWS>
 __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
                                             const int32_t* __restrict__ cu_q,
                                             const int32_t* __restrict__ cu_k, int qt, int G,
-                                            int w, int n_ranges, SplitCursor& c) {
+                                            int Hk, SplitCursor& c) {
   const int lane = threadIdx.x & 63;
   int Lq = 0, Lk = 0, cost = 0, incl = 0;
+  int chunks = 0;  // lane: of the decode rows
   auto load = [&](int cb) {  // lane: sequence cb + lane
     const int s = cb + lane;
     Lq = 0;
@@ -150,7 +170,11 @@ __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
     if (s < sa.n_seqs) {
       Lq = cu_q[s + 1] - cu_q[s];
       Lk = cu_k[s + 1] - cu_k[s];
-      NKV_DBG(w == 0 && (Lq < 0 || Lk < 0 || Lq > Lk), NKV_DEBUG_LENGTH);
+      NKV_DBG(blockIdx.x == 0 && (Lq < 0 || Lk < 0 || Lq > Lk), NKV_DEBUG_LENGTH);
+    }
+    if (ROWS && Lq == 1) {
+      chunks += (max(Lk, 0) + kChunk - 1) / kChunk;
+      Lq = 0;
     }
     cost = 0;
     for (int t = 0; t * qt < Lq; ++t)
@@ -161,9 +185,23 @@ __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
   int T = 0;
   for (int cb = 0; cb < sa.n_seqs; cb += 64) T += load(cb);
   c.T = T;
-  c.C = max((T + n_ranges - 1) / n_ranges, sa.min_range);
-  const int x = w * c.C;
+  int n_ranges = (int)gridDim.x / Hk;  // of each KV head
+  c.row_groups = 0;
+  if constexpr (ROWS) {  // shared out by cost, at least a range of each kind that there is
+    const int rows = __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63) * row_cost(F8) / 4;
+    if (rows > 0) {
+      const int r = (int)((float)n_ranges * (float)rows / (float)(rows + T) + 0.5f);
+      const int r_rows = T > 0 ? min(max(r, 1), n_ranges - 1) : n_ranges;
+      n_ranges -= r_rows;
+      c.row_groups = r_rows * Hk;
+    }
+    if ((int)blockIdx.x < c.row_groups) return false;
+  }
+  c.group = (int)blockIdx.x - c.row_groups;
+  c.C = max((T + n_ranges - 1) / max(n_ranges, 1), sa.min_range);
+  const int x = c.group / Hk * c.C;
   if (x >= T) return false;
+  c.x = x;
   c.x_end = x + c.C;
   int base = 0, cb = 0;
   int tot = load(0);
@@ -187,17 +225,15 @@ __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
   }
   c.q0 = cu_q[c.seq];
   c.kb0 = cu_k[c.seq];
-  c.s_lo = 0;
   return true;
 }
 
 // The unit after the current one (false at the end of the stream).
-template <int D, bool F8>
+template <bool ROWS>
 __device__ __forceinline__ bool split_next(const int32_t* __restrict__ cu_q,
                                            const int32_t* __restrict__ cu_k, int qt, int u1,
                                            SplitCursor& c) {
   c.u0 = u1;
-  c.s_lo = 0;
   if (u1 >= c.T) return false;
   if (++c.tile * qt < c.Lq) return true;
   c.tile = 0;
@@ -205,7 +241,7 @@ __device__ __forceinline__ bool split_next(const int32_t* __restrict__ cu_q,
     ++c.seq;
     c.q0 = cu_q[c.seq];
     c.Lq = cu_q[c.seq + 1] - c.q0;
-  } while (c.Lq <= 0);
+  } while (c.Lq <= (ROWS ? 1 : 0));
   c.kb0 = cu_k[c.seq];
   c.Lk = cu_k[c.seq + 1] - c.kb0;
   return true;
@@ -213,7 +249,9 @@ __device__ __forceinline__ bool split_next(const int32_t* __restrict__ cu_q,
 
 // One workgroup's work: a whole tile of a sequence (plain), or its range of the stream of
 // units, each unit's key steps [s_lo, s_end) of n_steps (SPLIT).
-template <bool F8, int D, bool H16, bool PAGED, bool SPLIT>
+// HP (SPLIT, paged): KV heads a wave of the decode rows reads at once, 0 for decode rows as
+// tiles of one query.
+template <bool F8, int D, bool H16, bool PAGED, bool SPLIT, int HP = 0>
 __device__ __forceinline__ void prefill_body(
     const bf16_t* __restrict__ q, int64_t q_row_stride, const void* __restrict__ k_cache,
     const void* __restrict__ v_cache, int64_t k_row_stride, int64_t v_row_stride,
@@ -237,7 +275,10 @@ __device__ __forceinline__ void prefill_body(
   constexpr int kRpl8 = 64 / kLpr8;        // F8: rows per load
   constexpr int kNl8 = 16 / kRpl8;         // F8: loads per wave per tile
   const int QT = prefill_tile_rows(D, F8) / G;  // queries per tile
-  __shared__ __attribute__((aligned(1024))) char ring[kStages * kStageB];
+  constexpr int kRowLds = 2 * decode_lds_elems<F8, HP == 0 ? 1 : HP, D>();  // bytes a wave
+  constexpr int kRingB = kStages * kStageB;
+  __shared__ __attribute__((aligned(1024))) char
+      ring[HP > 0 && 4 * kRowLds > kRingB ? 4 * kRowLds : kRingB];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -245,23 +286,32 @@ __device__ __forceinline__ void prefill_body(
   const int g4 = lane >> 4;
   const int col = lane & 15;
 
-  const int kvh = blockIdx.x % Hk;
-  const int rest = blockIdx.x / Hk;
   SplitCursor cur;
+  int kvh = blockIdx.x % Hk;
   if constexpr (SPLIT) {
     // no unit of this range is cut at its end, unless one below says so
     if (tid == 0) sa.desc[blockIdx.x] = i32x4_t{0, 0, 0, 0};
-    if (!split_begin<D, F8>(sa, cu_seqlens_q, cu_seqlens_k, QT, G, rest, (int)gridDim.x / Hk,
-                            cur))
+    if (!split_begin<D, F8, (HP > 0)>(sa, cu_seqlens_q, cu_seqlens_k, QT, G, Hk, cur)) {
+      if constexpr (HP > 0) {
+        if ((int)blockIdx.x < cur.row_groups)
+          decode_stream<F8, HP, D, H16>(
+              OneRowSeqs{cu_seqlens_q, cu_seqlens_k, sa.n_seqs}, (int)blockIdx.x * 4 + wave,
+              cur.row_groups * 4, reinterpret_cast<bf16_t*>(ring + wave * kRowLds), q,
+              q_row_stride, k_cache, v_cache, block_tables, bt_row_stride, Hk, G, sa.ncg,
+              block_size, max_blocks, n_limit, sa.min_chunks, scale_log2, v_scale, sa.row_part,
+              sa.row_desc);
+      }
       return;  // uniform
+    }
+    kvh = cur.group % Hk;
   } else {
+    const int rest = blockIdx.x / Hk;
     cur.tile = n_tiles - 1 - rest % n_tiles;  // largest tiles first
     cur.seq = rest / n_tiles;
     cur.q0 = cu_seqlens_q[cur.seq];
     cur.Lq = cu_seqlens_q[cur.seq + 1] - cur.q0;
     cur.kb0 = cu_seqlens_k[cur.seq];
     cur.Lk = cu_seqlens_k[cur.seq + 1] - cur.kb0;
-    cur.s_lo = 0;
   }
   int u1 = 0;        // the unit's end in the stream
   int snap = 0;      // a cut this near to the unit's ends moves there
@@ -292,11 +342,11 @@ __device__ __forceinline__ void prefill_body(
     const int sc = step_cost<D, F8>(min(QT, Lq - j0) * G);
     snap = kSnap * sc;
     u1 = cur.u0 + n_steps * sc;
-    const int x = rest * cur.C;  // the range's begin, which may lie in its first unit
-    if (x >= cur.u0 + snap) {
-      if (x > u1 - snap) continue;  // it belongs to the range before (the loop's condition
+    // the range's begin may lie in its first unit
+    if (cur.x >= cur.u0 + snap) {
+      if (cur.x > u1 - snap) continue;  // it belongs to the range before (the loop's condition
                                     // steps to the next unit)
-      s_lo = (x - cur.u0 + sc - 1) / sc;
+      s_lo = (cur.x - cur.u0 + sc - 1) / sc;
     }
     cut = false;
     if (cur.x_end < u1 && cur.x_end < cur.T) {  // the range ends within this unit
@@ -315,7 +365,7 @@ __device__ __forceinline__ void prefill_body(
   };
   auto describe = [&]() {
     const int w0 = (cur.u0 + snap + cur.C - 1) / cur.C;  // the unit's first cut
-    sa.desc[blockIdx.x] = i32x4_t{(u1 - snap) / cur.C - w0 + 2, q0 + j0, min(QT, Lq - j0), 0};
+    sa.desc[blockIdx.x] = i32x4_t{(u1 - snap) / cur.C - w0 + 2, q0 + j0, min(QT, Lq - j0), kvh};
   };
   const int k_lim = SPLIT ? min(Lk, s_end * kStep) : Lk;  // keys to load
 
@@ -750,7 +800,7 @@ __device__ __forceinline__ void prefill_body(
       *reinterpret_cast<uint2*>(op + db * 16) = w;
     }
   }
-  } while (SPLIT && !cut && split_next<D, F8>(cu_seqlens_q, cu_seqlens_k, QT, u1, cur));
+  } while (SPLIT && !cut && split_next<(HP > 0)>(cu_seqlens_q, cu_seqlens_k, QT, u1, cur));
 }
 
 #define NKV_PREFILL_PARAMS                                                                      \
@@ -771,33 +821,46 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void prefill_varlen_kernel(
   prefill_body<F8, D, H16, PAGED, false>(NKV_PREFILL_PASS, SplitArgs{});
 }
 
-template <bool F8, int D, bool H16, bool PAGED>
+template <bool F8, int D, bool H16, bool PAGED, int HP>
 __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void prefill_split_kernel(
     NKV_PREFILL_PARAMS, const SplitArgs sa) {
-  prefill_body<F8, D, H16, PAGED, true>(NKV_PREFILL_PASS, sa);
+  prefill_body<F8, D, H16, PAGED, true, HP>(NKV_PREFILL_PASS, sa);
 }
 
 // Merges the parts of the units that ranges cut: descriptor x (of the workgroup that holds a
 // unit's first part; part p > 0 is in the first slot of the workgroup p * Hk after it) and rows
-// 32*y .. of its tile. A wave merges four rows at once, lane l output dims N*l .. N*l+N-1, eight
+// 32*y .. of its tile (block y * groups + x). The blocks after those merge the decode rows'
+// partials, one (sequence, query head) a wave. A wave merges four rows at once, lane l output dims N*l .. N*l+N-1, eight
 // parts' loads in flight. Where the rows leave waves idle (a decode row's tile has G) they take
 // every n-th part each and merge once more through LDS.
 constexpr int kMergeRows = 32;
 constexpr int kMergeWaves = kMergeRows / 4;
 template <int D, bool H16>
 __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(
-    const i32x4_t* __restrict__ desc, const float* __restrict__ part, int32_t Hk, int32_t G,
-    int32_t tile_rows, float v_scale, bf16_t* __restrict__ out, int64_t out_row_stride) {
+    const SplitArgs sa, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k,
+    int32_t Hk, int32_t G, int32_t tile_rows, int32_t n_groups, float v_scale,
+    bf16_t* __restrict__ out, int64_t out_row_stride) {
   constexpr int N = D / 64;
   constexpr int kRow = prefill_part_row(D);
   __shared__ float so[kMergeWaves][4][N][64];
   __shared__ float2 sml[kMergeWaves][4];
-  const i32x4_t d = desc[blockIdx.x];
-  const int n_parts = d[0];
-  const int rows = d[2] * G;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int y0 = blockIdx.y * kMergeRows;
+  const int n_tile_blocks = (tile_rows + kMergeRows - 1) / kMergeRows * n_groups;
+  if ((int)blockIdx.x >= n_tile_blocks) {
+    const int Hq = Hk * G;
+    const int id = ((int)blockIdx.x - n_tile_blocks) * kMergeWaves + wave;
+    const int b = id / Hq;
+    if (b < sa.n_seqs && cu_q[b + 1] - cu_q[b] == 1)  // uniform over the wave
+      decode_combine<D, H16>(OneRowSeqs{cu_q, cu_k, sa.n_seqs}, b, id - b * Hq, Hq, Hk, sa.ncg,
+                             sa.row_part, sa.row_desc, out, out_row_stride);
+    return;
+  }
+  const int x = blockIdx.x % n_groups;
+  const i32x4_t d = sa.desc[x];
+  const int n_parts = d[0];
+  const int rows = d[2] * G;
+  const int y0 = (int)blockIdx.x / n_groups * kMergeRows;
   if (n_parts < 2 || y0 >= rows) return;  // uniform over the workgroup
   // groups of four rows, rounded up to a power of two, and the waves that share one's parts
   const int left = rows - y0;
@@ -806,8 +869,8 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(
   const int r0 = y0 + (wave % groups) * 4;
   const int share = wave / groups;
   const int64_t tile_f = (int64_t)tile_rows * kRow;
-  const float* first = part + ((int64_t)blockIdx.x * 2 + 1) * tile_f;
-  const float* next = part + (int64_t)blockIdx.x * 2 * tile_f;  // + p * 2 * Hk tiles
+  const float* first = sa.part + ((int64_t)x * 2 + 1) * tile_f;
+  const float* next = sa.part + (int64_t)x * 2 * tile_f;  // + p * 2 * Hk tiles
   float M[4], L[4], o[4][N];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -870,7 +933,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(
       }
     }
   }
-  const int kvh = blockIdx.x % Hk;
+  const int kvh = d[3];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = r0 + i;
@@ -888,22 +951,50 @@ namespace nkv {
 static int prefill_ranges(int32_t n_kv_heads, int32_t head_dim) {
   return std::max(1, device_cus() * (head_dim == 256 ? 1 : 2) / n_kv_heads);
 }
-static size_t prefill_split_bytes(int32_t n_kv_heads, int32_t head_dim, bool f8) {
-  const size_t groups = (size_t)prefill_ranges(n_kv_heads, head_dim) * n_kv_heads;
-  const size_t tile = (size_t)prefill_tile_rows(head_dim, f8) * prefill_part_row(head_dim);
-  return groups * (sizeof(i32x4_t) + 2 * tile * sizeof(float));
+// The split launch's workspace: a descriptor and two tiles of partial rows per workgroup; for
+// the decode rows a descriptor per (sequence, KV head, column group) and a partial row per
+// query head for every wave of a head group and every sequence.
+struct SplitSizes {
+  size_t groups, desc, part, row_desc, row_part;
+  size_t bytes() const { return desc + part + row_desc + row_part; }
+};
+static SplitSizes prefill_split_sizes(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads,
+                                      int32_t head_dim, bool f8) {
+  SplitSizes z;
+  z.groups = (size_t)prefill_ranges(n_kv_heads, head_dim) * n_kv_heads;
+  z.desc = z.groups * sizeof(i32x4_t);
+  const size_t row = prefill_part_row(head_dim) * sizeof(float);
+  z.part = z.groups * 2 * prefill_tile_rows(head_dim, f8) * row;
+  z.row_desc = (size_t)n_seqs * n_kv_heads * decode_ncg(n_q_heads / n_kv_heads) *
+               sizeof(i32x4v_t);
+  // waves of a head group x Hq <= 4 * groups x its columns (at most 16)
+  z.row_part = (4 * z.groups * std::min(kMaxCols, n_q_heads) + (size_t)n_seqs * n_q_heads) * row;
+  return z;
+}
+// KV heads a wave of the decode rows reads at once: up to a 512-byte piece of every row, as the
+// decode kernel's plan takes them for batches that fill the chip (a step that has prompts too
+// is long enough for it).
+template <bool F8>
+static int prefill_row_heads(int32_t n_kv_heads, int32_t G, int32_t head_dim) {
+  const int most = head_dim == 256 ? (F8 ? 2 : 1) : (F8 && head_dim == 128 ? 4 : 2);
+  for (int hp = most; hp > 1; hp /= 2)
+    if (n_kv_heads % hp == 0 && hp * G <= kMaxCols) return hp;
+  return 1;
 }
 
-// Whether the split launch is the faster one, from what the host knows: the longest sequence,
-// the rows of q and how many sequences share them. Plain, the workgroup of the longest
-// sequence's last tile walks its keys alone, 1.9 us a 64-key step, however few tiles there are.
-// Split, every workgroup has an equal share, 2.2 us a step with the chip full, and the launch,
-// the parts' writing and the merge add 35 us. The steps of a batch are taken as half of the
-// longest sequence's per tile; one sequence's are known. Both sides measured on 110 random
-// steps of 1 - 104 sequences, 1 - 3000 new tokens and contexts of up to 16k: the rule's choice
-// was never slower than the plain launch, up to 4.0x faster, and lost 0.9% against always
-// knowing the faster (three steps, near the line). Chunk of 512 on 12288 tokens (Hq 32, Hk 8):
-// 337 -> 138 us; 48 decode rows with two 512-token chunks: 208 -> 138 us.
+// Whether the split launch is the faster one, from what the host knows: the longest lengths, the
+// rows of q and how many sequences share them (with as few prompts as could bring them, the
+// others being decode rows). In us, on times fitted to both sides of 130 random steps (1 - 104
+// sequences, 1 - 3000 new tokens, contexts of up to 16k, every KV type):
+//  * plain, the workgroup of the longest sequence's last tile walks its keys alone, 1.7 a 64-key
+//    step, however few tiles there are; with many decode rows each takes a tile's time, 6 a step
+//    for as many as the chip holds;
+//  * split, every workgroup has an equal share: 2.8 a step of the tiles and 1 of the rows (their
+//    bytes), and 35 for the launch, the parts' writing and the merge.
+// The keys of a batch are taken as half of the longest sequence's. The rule's choice was at most
+// 7% slower than the plain launch (one step of 130), up to 4.9x faster, and lost 0.7% against
+// always knowing the faster. 512 tokens on 12288 (Hq 32, Hk 8): 338 -> 138 us; 48 decode rows
+// with two 512-token chunks: 208 -> 117 us.
 static bool prefill_split_wins(int32_t n_seqs, int64_t total_q, int32_t max_seqlen_q,
                                int32_t max_seqlen_k, int32_t n_q_heads, int32_t n_kv_heads,
                                int32_t head_dim, bool f8) {
@@ -913,14 +1004,22 @@ static bool prefill_split_wins(int32_t n_seqs, int64_t total_q, int32_t max_seql
   // every range counts the tiles of the sequences before it: not for long prompts (whose
   // tiles fill the chip anyway)
   if (tiles_max > 96 || max_seqlen_k < max_seqlen_q) return false;
-  const int64_t tiles = std::min(n_seqs * tiles_max, total_q / qt + n_seqs);
+  const int64_t more = std::max<int64_t>(0, total_q - n_seqs);  // beyond one token each
+  const int64_t prompts =
+      max_seqlen_q > 1 ? std::min<int64_t>(n_seqs, (more + max_seqlen_q - 2) / (max_seqlen_q - 1))
+                       : 0;
+  const int64_t rows = n_seqs - prompts;
+  const int64_t tiles = std::min(prompts * tiles_max, (total_q - rows) / qt + prompts);
   const double steps = (max_seqlen_k + kStep - 1) / kStep;
-  const double seen = n_seqs == 1 ? 1.0 - 0.5 * max_seqlen_q / max_seqlen_k : 0.5;
-  const double share = tiles * steps * seen / prefill_ranges(n_kv_heads, head_dim);
   // positions of the stream are 32 bits
-  if (tiles * steps * 8 >= 2147483648.0) return false;
+  if ((tiles + rows) * steps * 8 >= 2147483648.0) return false;
+  const double per_range = 1.0 / prefill_ranges(n_kv_heads, head_dim);
+  const double seen = 1.0 - 0.5 * max_seqlen_q / max_seqlen_k;  // causal: of a prompt's own keys
+  const double tile_steps = tiles * steps * seen * per_range * (n_seqs == 1 ? 1.0 : 0.5);
+  const double row_steps = rows * steps * 0.5 * per_range;
   const double dim = head_dim / 128.0;
-  return 1.9 * dim * steps > 35.0 + 2.2 * dim * share;
+  return dim * std::max(1.7 * steps, 2.5 * tile_steps + 6.0 * row_steps) >
+         35.0 + dim * (2.8 * tile_steps + row_steps);
 }
 
 // `split`: a split launch over `workspace`; a plain one otherwise.
@@ -982,38 +1081,69 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
   const int n_tiles = (max_seqlen_q + qt - 1) / qt;
   const float sl2 = scale * k_scale * kLog2e;
   int64_t grid = (int64_t)n_seqs * n_tiles * n_kv_heads;
+  int64_t merge_grid = 0;
+  int row_heads = 0;
   SplitArgs sa = {};
   if (split) {
-    const size_t need = prefill_split_bytes(n_kv_heads, head_dim, F8);
+    const SplitSizes z = prefill_split_sizes(n_seqs, n_q_heads, n_kv_heads, head_dim, F8);
+    const size_t need = z.bytes();
     NKV_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= need, NKV_EWORKSPACE,
                 "%s: the split launch needs a 16-byte aligned workspace of %zu bytes (got %zu)",
                 what, need, workspace_bytes);
-    grid = (int64_t)prefill_ranges(n_kv_heads, head_dim) * n_kv_heads;
+    grid = (int64_t)z.groups;
     sa.n_seqs = n_seqs;
     sa.min_range = kMinRange;
-    sa.desc = static_cast<i32x4_t*>(workspace);
-    sa.part = reinterpret_cast<float*>(sa.desc + grid);
+    char* ws = static_cast<char*>(workspace);
+    sa.desc = reinterpret_cast<i32x4_t*>(ws);
+    sa.part = reinterpret_cast<float*>(ws + z.desc);
+    sa.row_desc = reinterpret_cast<i32x4v_t*>(ws + z.desc + z.part);
+    sa.row_part = reinterpret_cast<float*>(ws + z.desc + z.part + z.row_desc);
+    sa.ncg = decode_ncg(g);
+    sa.min_chunks = block_tables ? decode_min_chunks(max_blocks, block_size) : 0;
+    // a range for each kind of work, dense cache rows, and positions of the decode rows' chunks
+    // in 32 bits
+    if (block_tables && prefill_ranges(n_kv_heads, head_dim) >= 2 &&
+        k_row_stride == (int64_t)n_kv_heads * head_dim &&
+        (int64_t)max_blocks * block_size < (1ll << 30) &&
+        (int64_t)block_size * k_row_stride * kEl < (1ll << 31))
+      row_heads = prefill_row_heads<F8>(n_kv_heads, g, head_dim);
+    merge_grid = grid * ((tile_rows + kMergeRows - 1) / kMergeRows) +
+                 (row_heads ? ((int64_t)n_seqs * n_q_heads + kMergeWaves - 1) / kMergeWaves : 0);
+    NKV_REQUIRE(merge_grid < (1ll << 31), NKV_EUNSUPPORTED, "%s: grid too large", what);
   }
   NKV_REQUIRE(grid < (1ll << 31), NKV_EUNSUPPORTED, "%s: grid too large", what);
 #define NKV_PREFILL_ARGS                                                                       \
   (const bf16_t*)q, q_row_stride, k_cache, v_cache, k_row_stride, v_row_stride, cu_seqlens_q,  \
       cu_seqlens_k, block_tables, bt_row_stride, n_kv_heads, g, block_size, max_blocks,        \
       n_limit, n_tiles, sl2, v_scale, (bf16_t*)out, out_row_stride
+#define NKV_PREFILL_SPLIT(D, P, HP)                                                            \
+  hipLaunchKernelGGL((prefill_split_kernel<F8, D, H16, P, HP>), dim3((unsigned)grid), dim3(256), \
+                     0, as_stream(stream), NKV_PREFILL_ARGS, sa)
 #define NKV_PREFILL_LAUNCH_P(D, P)                                                             \
   do {                                                                                         \
-    if (split) {                                                                               \
-      hipLaunchKernelGGL((prefill_split_kernel<F8, D, H16, P>), dim3((unsigned)grid),          \
-                         dim3(256), 0, as_stream(stream), NKV_PREFILL_ARGS, sa);               \
-      hipLaunchKernelGGL((prefill_merge_kernel<D, H16>),                                       \
-                         dim3((unsigned)grid, (unsigned)(tile_rows + kMergeRows - 1) /         \
-                                                  kMergeRows),                                 \
-                         dim3(64 * kMergeWaves), 0, as_stream(stream), sa.desc, sa.part,       \
-                         n_kv_heads, g,                                                        \
-                         tile_rows, v_scale, (bf16_t*)out, out_row_stride);                    \
-    } else {                                                                                   \
+    if (!split) {                                                                              \
       hipLaunchKernelGGL((prefill_varlen_kernel<F8, D, H16, P>), dim3((unsigned)grid),         \
                          dim3(256), 0, as_stream(stream), NKV_PREFILL_ARGS);                   \
+      break;                                                                                   \
     }                                                                                          \
+    if constexpr (P) {                                                                         \
+      if (row_heads == 0) NKV_PREFILL_SPLIT(D, P, 0);                                          \
+      else if (row_heads == 1) NKV_PREFILL_SPLIT(D, P, 1);                                     \
+      else if constexpr (D < 256 || F8) {                                                      \
+        if constexpr (D == 128 && F8) {                                                        \
+          if (row_heads == 4) NKV_PREFILL_SPLIT(D, P, 4);                                      \
+          else NKV_PREFILL_SPLIT(D, P, 2);                                                     \
+        } else {                                                                               \
+          NKV_PREFILL_SPLIT(D, P, 2);                                                          \
+        }                                                                                      \
+      }                                                                                        \
+    } else {                                                                                   \
+      NKV_PREFILL_SPLIT(D, P, 0);                                                              \
+    }                                                                                          \
+    hipLaunchKernelGGL((prefill_merge_kernel<D, H16>), dim3((unsigned)merge_grid),             \
+                       dim3(64 * kMergeWaves), 0, as_stream(stream), sa, cu_seqlens_q,         \
+                       cu_seqlens_k, n_kv_heads, g, tile_rows, (int32_t)grid, v_scale,         \
+                       (bf16_t*)out, out_row_stride);                                          \
   } while (0)
 #define NKV_PREFILL_LAUNCH(D)                                                                  \
   do {                                                                                         \
@@ -1025,6 +1155,7 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
   else NKV_PREFILL_LAUNCH(256);
 #undef NKV_PREFILL_LAUNCH
 #undef NKV_PREFILL_LAUNCH_P
+#undef NKV_PREFILL_SPLIT
 #undef NKV_PREFILL_ARGS
   return check_launch(F8 ? "nkv_prefill_varlen_fp8"
                          : H16 ? "nkv_prefill_varlen_f16" : "nkv_prefill_varlen");
@@ -1084,11 +1215,15 @@ extern "C" int nkv_prefill_varlen_fp8(const void* q, int64_t q_row_stride, const
                                    out, out_row_stride, stream);
 }
 
-extern "C" size_t nkv_prefill_split_workspace_bytes(int32_t n_q_heads, int32_t n_kv_heads,
-                                                    int32_t head_dim, int32_t kv_type) {
+extern "C" size_t nkv_prefill_split_workspace_bytes(int32_t n_seqs, int32_t n_q_heads,
+                                                    int32_t n_kv_heads, int32_t head_dim,
+                                                    int32_t kv_type) {
   using namespace nkv;
-  if (n_q_heads <= 0 || n_kv_heads <= 0 || !prefill_dim_ok(head_dim)) return 0;
-  return prefill_split_bytes(n_kv_heads, head_dim, kv_type == NKV_KV_FP8);
+  if (n_seqs <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_q_heads % n_kv_heads != 0 ||
+      !prefill_dim_ok(head_dim))
+    return 0;
+  return prefill_split_sizes(n_seqs, n_q_heads, n_kv_heads, head_dim, kv_type == NKV_KV_FP8)
+      .bytes();
 }
 
 extern "C" size_t nkv_prefill_split_plan(int32_t n_seqs, int64_t total_q, int32_t max_seqlen_q,
@@ -1103,7 +1238,7 @@ extern "C" size_t nkv_prefill_split_plan(int32_t n_seqs, int64_t total_q, int32_
   const bool f8 = kv_type == NKV_KV_FP8;
   return prefill_split_wins(n_seqs, total_q, max_seqlen_q, max_seqlen_k, n_q_heads, n_kv_heads,
                             head_dim, f8)
-             ? prefill_split_bytes(n_kv_heads, head_dim, f8)
+             ? prefill_split_sizes(n_seqs, n_q_heads, n_kv_heads, head_dim, f8).bytes()
              : 0;
 }
 

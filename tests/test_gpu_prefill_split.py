@@ -22,6 +22,8 @@ MIXES = {
     "edges": [(47, 63), (48, 64), (49, 65), (96, 128), (97, 1281)],
     # a sequence per range and more than one batch of 64 sequences
     "many": [(1 + i % 3, 30 * (i % 7) + 3) for i in range(130)],
+    # decode rows alone, more than one batch of 64 of them
+    "rows": [(1, 17 * (i % 40) + 1) for i in range(90)],
     # one chunk on a long prefix
     "chunk": [(130, 2311)],
 }
@@ -60,7 +62,7 @@ def _split(dev, q, k, v, cu_q, cu_k, bt, kind, scale):
     # a strided V stays strided on the device
     vd = v.to(dev) if v.is_contiguous() else \
         torch.empty_strided(v.shape, v.stride(), dtype=v.dtype, device=dev).copy_(v)
-    nbytes = L.lib().nkv_prefill_split_workspace_bytes(Hq, Hk, D, t)
+    nbytes = L.lib().nkv_prefill_split_workspace_bytes(cu_q.numel() - 1, Hq, Hk, D, t)
     ws = torch.full((nbytes,), 0xff, dtype=torch.uint8, device=dev)  # NaN where nothing is written
     out = torch.full((N, Hq, D), float("nan"), dtype=q.dtype, device=dev)
     max_q = int((cu_q[1:] - cu_q[:-1]).max())
@@ -92,6 +94,9 @@ def _split(dev, q, k, v, cu_q, cu_k, bt, kind, scale):
     ("edges", 32, 8, 128, "fp16", 0, False),
     ("many", 8, 4, 128, "bf16", 16, True),
     ("many", 8, 2, 128, "fp8", 64, True),
+    ("rows", 32, 8, 128, "bf16", 256, True),
+    ("rows", 24, 1, 128, "fp16", 16, True),     # two column groups of query heads
+    ("rows", 8, 4, 64, "bf16", 64, True),
     ("chunk", 32, 8, 128, "bf16", 256, True),
     ("chunk", 8, 1, 64, "fp16", 0, False),
 ])
@@ -103,6 +108,23 @@ def test_split_matches_the_oracle(dev, mix, Hq, Hk, D, kind, B, paged):
     ref = varlen_prefill_ref(q.float(), k.float() * s, v.float() * s, cu_q, cu_k, D ** -0.5,
                              block_tables=bt)
     assert (out.float().cpu() - ref).abs().max().item() <= TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+def test_split_takes_invalid_blocks_as_zero_keys(nkv, dev, kind):
+    """Table entries outside the pool, and keys past the table's width, are zero keys that take
+    their weight, in the decode rows' stream too: the plain launch's results (two orders of
+    the same sums, outputs rounded to bf16: 2^-8 of |out| < 4)."""
+    mix = [(1, 700), (1, 300), (60, 500), (1, 200)]
+    q, k, v, cu_q, cu_k, bt = _inputs(dev, mix, 16, 4, 128, kind, 64, True, seed=8)
+    bt[0, 3], bt[1, 0], bt[2, 2], bt[3, 1] = -1, 10 ** 6, -7, -1
+    bt = bt[:, :10].contiguous()  # row 0's last key block is past the table
+    out = _split(dev, q, k, v, cu_q, cu_k, bt, kind, 128 ** -0.5)
+    s = 1 / 16 if kind == "fp8" else 1.0
+    plain = nkv.varlen_prefill(*(x.to(dev) for x in (q, k, v, cu_q, cu_k)), 60, 128 ** -0.5,
+                               block_tables=bt.to(dev), k_scale=s, v_scale=s)
+    assert (out.float() - plain.float()).abs().max().item() <= 2 ** -6
 
 
 @pytest.mark.gpu
@@ -140,9 +162,10 @@ def test_split_plan_and_arguments_on_the_host():
     """The rule, and what the entry point refuses, without a GPU."""
     lib = L.lib()
     plan = lambda *a: lib.nkv_prefill_split_plan(*a)  # noqa: E731
-    full = lib.nkv_prefill_split_workspace_bytes(32, 8, 128, L.NKV_KV_BF16)
+    size = lambda n: lib.nkv_prefill_split_workspace_bytes(n, 32, 8, 128, L.NKV_KV_BF16)  # noqa: E731
+    full = size(1)
     assert plan(1, 512, 512, 12800, 32, 8, 128, L.NKV_KV_BF16) == full > 0
-    assert plan(50, 1072, 512, 5700, 32, 8, 128, L.NKV_KV_BF16) == full
+    assert plan(50, 1072, 512, 5700, 32, 8, 128, L.NKV_KV_BF16) == size(50) > full
     # tiles that fill the chip, short contexts, prompts of many tiles, nothing known
     assert plan(16, 32768, 2048, 9000, 32, 8, 128, L.NKV_KV_BF16) == 0
     assert plan(3, 120, 40, 300, 32, 8, 128, L.NKV_KV_BF16) == 0
