@@ -354,6 +354,50 @@ int nkv_prefill_varlen_split(int32_t kv_type, const void* q, int64_t q_row_strid
                              float k_scale, float v_scale, void* out, int64_t out_row_stride,
                              void* workspace, size_t workspace_bytes, void* stream);
 
+/* One layer's call of a step, Attention.forward's store and attention in one entry point: the
+ * new rows' store (nkv_store_kvcache or nkv_store_kvcache_fp8, by kv_type), then
+ * nkv_paged_decode (decode != 0: cu_or_lens = context_lens, cu_seqlens_k and max_seqlen_q
+ * unused, the workspace of nkv_paged_decode_workspace_bytes) or the paged variable-length
+ * attention (cu_or_lens = cu_seqlens_q; split over a workspace of nkv_prefill_split_plan's
+ * bytes, plain with workspace_bytes = 0). Every argument as in those; caches dense. Returns
+ * NKV_EWORKSPACE for a decode workspace that is too small before anything is launched.
+ * Replaces: Attention.forward, nanokvllm/layers/attention.py:67-108. */
+typedef struct nkv_attention_args {
+  const void* q;
+  int64_t q_row_stride;
+  const void* key;
+  int64_t key_row_stride;
+  const void* value;
+  int64_t value_row_stride;
+  void* k_cache;
+  void* v_cache;
+  const int32_t* slot_mapping;
+  int64_t n_tokens; /* new rows */
+  const int32_t* block_tables;
+  int64_t bt_row_stride;
+  int64_t max_blocks_per_seq;
+  const int32_t* cu_or_lens;
+  const int32_t* cu_seqlens_k;
+  int64_t n_seqs;
+  int64_t max_seqlen_q;
+  int64_t n_q_heads;
+  int64_t n_kv_heads;
+  int64_t head_dim;
+  int64_t block_size;
+  int64_t n_blocks;
+  int64_t kv_type; /* NKV_KV_* */
+  int64_t decode;
+  void* out;
+  int64_t out_row_stride;
+  void* workspace;
+  int64_t workspace_bytes;
+  void* stream;
+  double scale;
+  double k_scale; /* fp8 */
+  double v_scale;
+} nkv_attention_args;
+int nkv_attention(const nkv_attention_args* args);
+
 /* Aggregation of key importance over query heads (compression scoring). */
 #define NKV_AGG_ALL 0   /* sum over all Hq heads -> one kept set per sequence
                            (nanokvllm/layers/CompressMethod.py:41-42) */

@@ -20,6 +20,7 @@ LIB_PATH = os.path.join(PKG_DIR, "libnkv_amd.so")
 DEBUG_LIB_PATH = os.path.join(PKG_DIR, "libnkv_amd_debug.so")
 
 NKV_OK = 0
+NKV_EWORKSPACE = -3
 NKV_KV_BF16 = 0
 NKV_KV_F16 = 1
 NKV_KV_FP8 = 2
@@ -80,6 +81,7 @@ SIGNATURES = {
     "nkv_prefill_varlen_split": (C.c_int, [_i32, _p, _i64, _p, _p, _i64, _i64, _p, _p, _p, _i64,
                                            _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i64, _f32,
                                            _f32, _f32, _p, _i64, _p, _sz, _p]),
+    "nkv_attention": (C.c_int, [C.c_char_p]),  # the packed nkv_attention_args
     "nkv_compress_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32]),
     "nkv_compress_score": (C.c_int, [_p, _i64, _p, _p, _i64, _i32, _p, _p, _i32, _i32, _i32, _i32,
                                      _i32, _i32, _i64, _f32, _i32, _p, _p, _sz, _p]),
@@ -197,7 +199,7 @@ def need(cond: bool, msg: str) -> None:
 
 def stream_of(t: torch.Tensor) -> int:
     """HIP stream handle of torch's current stream on t's device."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
