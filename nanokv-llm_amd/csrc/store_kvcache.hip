@@ -9,14 +9,20 @@
 // any store, lanes of a wave cover consecutive chunks of one row so every
 // wave-wide load/store is a coalesced 1 KiB access, and a bounded grid strides
 // over the rest (prefill-sized token counts keep ~128 KiB in flight per CU).
+// Up to about 16k tokens (Hk 8) it is one chunk a thread, so that four times the waves share
+// them, with 32-bit index arithmetic (four 64-bit divisions a thread took longer than a decode
+// step's loads): 64 tokens 3.5 -> 2.7 us, 512 3.8 -> 2.8, 4096 6.7 -> 5.5, 9000 13.6 -> 12.9;
+// 38000 with four chunks a thread 52.3 (6.0 TB/s), with one 52.6.
 #include "nkv_common.h"
 
 namespace nkv {
 
 constexpr int kStoreThreads = 256;
-constexpr int kUnroll = 4;
+constexpr int kStoreUnroll = 4;
+constexpr int kStoreFewGroups = 16384;  // one chunk a thread up to this many workgroups of them
 
-template <typename Chunk>
+// Index: uint32_t where the chunks fit, else uint64_t.
+template <typename Chunk, int kUnroll, typename Index>
 __global__ __launch_bounds__(kStoreThreads) void store_kvcache_kernel(
     const char* __restrict__ key, int64_t key_stride_b,
     const char* __restrict__ value, int64_t value_stride_b,
@@ -24,24 +30,24 @@ __global__ __launch_bounds__(kStoreThreads) void store_kvcache_kernel(
     const int32_t* __restrict__ slot_mapping, int64_t n_tokens,
     int32_t chunks_per_row, int64_t n_slots) {
   const int64_t row_bytes = (int64_t)chunks_per_row * sizeof(Chunk);
-  const int64_t per_token = 2 * (int64_t)chunks_per_row;
-  const int64_t n_items = n_tokens * per_token;
-  const int64_t span = (int64_t)kStoreThreads * kUnroll;
-  for (int64_t base = (int64_t)blockIdx.x * span; base < n_items;
-       base += (int64_t)gridDim.x * span) {
+  const Index per_token = 2 * (Index)chunks_per_row;
+  const Index n_items = (Index)n_tokens * per_token;
+  const Index span = (Index)kStoreThreads * kUnroll;
+  for (Index base = (Index)blockIdx.x * span; base < n_items; base += (Index)gridDim.x * span) {
     Chunk val[kUnroll];
     int64_t dst[kUnroll];  // byte offset of the destination chunk, -1 = skip
     bool is_v[kUnroll];
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
-      const int64_t i = base + (int64_t)u * kStoreThreads + threadIdx.x;
+      const Index i = base + (Index)u * kStoreThreads + threadIdx.x;
       const bool ok = i < n_items;
-      const int64_t ic = ok ? i : 0;
-      const int64_t tok = ic / per_token;
-      const int64_t r = ic - tok * per_token;
-      is_v[u] = r >= chunks_per_row;
-      const int64_t c = is_v[u] ? r - chunks_per_row : r;
-      const char* src = is_v[u] ? value + tok * value_stride_b : key + tok * key_stride_b;
+      const Index ic = ok ? i : 0;
+      const Index tok = ic / per_token;
+      const Index r = ic - tok * per_token;
+      is_v[u] = r >= (Index)chunks_per_row;
+      const Index c = is_v[u] ? r - (Index)chunks_per_row : r;
+      const char* src = is_v[u] ? value + (int64_t)tok * value_stride_b
+                                : key + (int64_t)tok * key_stride_b;
       val[u] = reinterpret_cast<const Chunk*>(src)[c];
       const int64_t slot = slot_mapping[tok];
       // -1 = padding; slots outside the cache are skipped
@@ -84,19 +90,27 @@ extern "C" int nkv_store_kvcache(const void* key, int64_t key_row_stride,
                    aligned16(k_cache) && aligned16(v_cache);
   const int32_t cpr = (int32_t)(vec ? row_bytes / 16 : row_bytes / 2);
   const int64_t n_items = n_tokens * 2 * cpr;
-  const int64_t spans = (n_items + kStoreThreads * kUnroll - 1) / (kStoreThreads * kUnroll);
+  const bool few = n_items <= (int64_t)kStoreThreads * kStoreFewGroups;
+  const int64_t span = (int64_t)kStoreThreads * (few ? 1 : kStoreUnroll);
+  const int64_t spans = (n_items + span - 1) / span;
   const unsigned grid = (unsigned)(spans < 4096 ? spans : 4096);
+  // 32-bit indexes run at most one grid's span past the last chunk
+  const bool small = n_items < (1ll << 31);
   hipStream_t s = as_stream(stream);
+#define NKV_STORE(CHUNK, UNROLL, INDEX)                                                        \
+  hipLaunchKernelGGL((store_kvcache_kernel<CHUNK, UNROLL, INDEX>), dim3(grid),                 \
+                     dim3(kStoreThreads), 0, s, (const char*)key, key_row_stride * 2,          \
+                     (const char*)value, value_row_stride * 2, (char*)k_cache, (char*)v_cache, \
+                     slot_mapping, n_tokens, cpr, n_slots)
   if (vec) {
-    hipLaunchKernelGGL(store_kvcache_kernel<uint4>, dim3(grid), dim3(kStoreThreads), 0, s,
-                       (const char*)key, key_row_stride * 2, (const char*)value,
-                       value_row_stride * 2, (char*)k_cache, (char*)v_cache, slot_mapping,
-                       n_tokens, cpr, n_slots);
+    if (few) NKV_STORE(uint4, 1, uint32_t);
+    else if (small) NKV_STORE(uint4, kStoreUnroll, uint32_t);
+    else NKV_STORE(uint4, kStoreUnroll, uint64_t);
   } else {
-    hipLaunchKernelGGL(store_kvcache_kernel<uint16_t>, dim3(grid), dim3(kStoreThreads), 0, s,
-                       (const char*)key, key_row_stride * 2, (const char*)value,
-                       value_row_stride * 2, (char*)k_cache, (char*)v_cache, slot_mapping,
-                       n_tokens, cpr, n_slots);
+    if (few) NKV_STORE(uint16_t, 1, uint32_t);
+    else if (small) NKV_STORE(uint16_t, kStoreUnroll, uint32_t);
+    else NKV_STORE(uint16_t, kStoreUnroll, uint64_t);
   }
+#undef NKV_STORE
   return check_launch("nkv_store_kvcache");
 }
