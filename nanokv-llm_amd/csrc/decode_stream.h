@@ -12,7 +12,9 @@ namespace nkv {
 
 constexpr int kChunk = 16;               // tokens per pipeline stage
 constexpr int kMinChunks = 4;            // minimum chunks per wave range
-constexpr int kMaxSlots = 128;           // partials per (sequence, query head) at most
+// partials per (sequence, query head) at most: what four waves' combine has in flight at once
+// (4 x 32), and one, so that a table of 512 chunks splits into ranges of 4
+constexpr int kMaxSlots = 129;
 constexpr int kWinBlocks = 64;           // block ids held per window (one per lane)
 constexpr int kBufferFlags = 0x00020000; // raw buffer resource word 3 (dword data)
 constexpr int kStreamPolicy = 2;         // cache policy "nt": K/V are read exactly once
@@ -33,7 +35,7 @@ typedef int32_t i32x4v_t __attribute__((ext_vector_type(4)));
 // Partial slots per (sequence, query head): a segment of n chunks is touched by at most
 // ceil(n / C) + 1 waves, and the kernel takes C >= decode_min_chunks, which is at least
 // kMinChunks and at least max_chunks / (slots - 1), so no segment has more than kMaxSlots
-// partials (the combine holds up to 128, two per lane).
+// partials (as many as the combine holds).
 static inline int64_t decode_slots(int32_t max_blocks, int32_t block_size) {
   const int64_t max_chunks = ((int64_t)max_blocks * block_size + kChunk - 1) / kChunk;
   const int64_t s = (max_chunks + kMinChunks - 1) / kMinChunks + 1;
@@ -82,14 +84,18 @@ struct OneRowSeqs {
   __device__ __forceinline__ int64_t row(int s) const { return cu_q[s]; }
 };
 
+// Chunks of a sequence of ctx keys.
+template <typename Seqs>
+__device__ __forceinline__ int seq_chunks(int ctx, int max_tokens) {
+  if constexpr (!Seqs::kZeroInvalid) NKV_DBG(ctx < 0 || ctx > max_tokens, NKV_DEBUG_LENGTH);
+  const int n = Seqs::kZeroInvalid ? ctx : min(ctx, max_tokens);
+  return n > 0 ? (n + kChunk - 1) / kChunk : 0;
+}
 template <typename Seqs>
 __device__ __forceinline__ void seq_load(SeqCursor& c, const Seqs& seqs, int max_tokens) {
   const int s = c.cb + (int)(threadIdx.x & 63);
   c.ctx = s < seqs.batch ? seqs.keys(s) : 0;
-  if constexpr (!Seqs::kZeroInvalid)
-    NKV_DBG(c.ctx < 0 || c.ctx > max_tokens, NKV_DEBUG_LENGTH);
-  const int n = Seqs::kZeroInvalid ? c.ctx : min(c.ctx, max_tokens);
-  c.nc = n > 0 ? (n + kChunk - 1) / kChunk : 0;
+  c.nc = seq_chunks<Seqs>(c.ctx, max_tokens);
   c.incl = wave_incl_scan(c.nc);
   c.tot = __builtin_amdgcn_readlane(c.incl, 63);
 }
@@ -189,11 +195,19 @@ __device__ __forceinline__ void decode_stream(
   // partial rows of this head group: (wave + sequence) x HPG columns, after the groups of
   // the query heads before qh0 (so the groups' regions add up to (waves + batch) x Hq rows)
   float* gpart = part + (int64_t)(Wh + batch) * qh0 * kPartRow;
+  // chunks of the whole batch: its lengths' loads in flight together, one reduction (the first
+  // 64 sequences' cursor is loaded with them)
   SeqCursor cur;
-  int T = 0;
-  for (cur.cb = 0; cur.cb < batch; cur.cb += 64) {
-    seq_load(cur, seqs, max_tokens);
-    T += cur.tot;
+  cur.cb = 0;
+  cur.base = 0;
+  seq_load(cur, seqs, max_tokens);
+  int T = cur.tot;
+  if (batch > 64) {
+    int more = 0;
+#pragma unroll 4
+    for (int s = 64 + lane; s < batch; s += 64)
+      more += seq_chunks<Seqs>(seqs.keys(s), max_tokens);
+    T += __builtin_amdgcn_readlane(wave_incl_scan(more), 63);
   }
   // equal ranges over the resident waves, at least min_chunks (which keeps every
   // segment within its partial slots)
@@ -201,9 +215,6 @@ __device__ __forceinline__ void decode_stream(
   const int k_begin = wi * C;
   if (k_begin >= T) return;
   const int k_end = min(T, k_begin + C);
-  cur.cb = 0;
-  cur.base = 0;
-  seq_load(cur, seqs, max_tokens);
 
   // per-lane load offset: lane l reads 16 bytes of row l / kLpr (+ kRpl per
   // load), byte 16 * (l % kLpr) of the wave's piece of the row; it stages them
@@ -446,8 +457,12 @@ __device__ __forceinline__ void decode_stream(
 }
 
 // Merge the partials of one (sequence, query head): O = sum_s 2^(m_s-M) O_s /
-// sum_s 2^(m_s-M) l_s. One wave per pair; lane l owns output dims N*l .. N*l+N-1.
-template <int D, bool H16, typename Seqs>
+// sum_s 2^(m_s-M) l_s. Lane l owns output dims N*l .. N*l+N-1. WAVES = 1: the calling wave
+// alone. WAVES > 1: the waves of a workgroup share the partials, wave w those with
+// s % WAVES == w (in its lane s / WAVES), and merge once more through LDS: a context that many
+// waves shared has up to kMaxSlots, and one wave took 10.3 us over the 120 of a 23001-token sequence
+// (a round trip for every eight rows), four waves with 32 rows in flight each 4.2 us.
+template <int D, bool H16, int WAVES, typename Seqs>
 __device__ __forceinline__ void decode_combine(
     const Seqs seqs, const int b, const int h, int32_t Hq, int32_t Hk, int32_t NCG,
     const float* __restrict__ part, const i32x4v_t* __restrict__ desc,
@@ -455,11 +470,13 @@ __device__ __forceinline__ void decode_combine(
   static_assert(decode_dim_ok(D), "head_dim 64, 128 or 256");
   constexpr int N = D / 64;
   constexpr int kPartRow = part_row(D);
+  constexpr int kPer = (kMaxSlots + 64 * WAVES - 1) / (64 * WAVES);  // (m, l) pairs a lane holds
+  constexpr int kFirst = WAVES > 1 ? 32 : 16;  // rows in flight with the (m, l) pairs
   const int lane = threadIdx.x & 63;
+  const int wave = WAVES > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
   const int G = Hq / Hk;
   // The context length and the KV head's descriptor first (one round trip), then every
-  // (m, l) pair and the first eight partial rows at once (the second).
-  static_assert(kMaxSlots <= 128, "two partials per lane");
+  // (m, l) pair and the first partial rows at once (the second).
   const int ctx = seqs.keys(b);
   const int hq = h % G;                         // query head within the KV head's group
   const int cg = NCG > 1 ? hq / kMaxCols : 0;    // its column group (0 unless G > 16)
@@ -469,20 +486,27 @@ __device__ __forceinline__ void decode_combine(
 #pragma unroll
   for (int i = 0; i < N; ++i) o[i] = 0.f;
   // the descriptor is written by this call for every sequence with ctx > 0
-  const int ns = ctx > 0 ? min(d.y, kMaxSlots) : 0;
-  if (ns == 0) {
-    store_dims<N, H16>(op, o, 0.f);
+  const int n_all = ctx > 0 ? min(d.y, kMaxSlots) : 0;
+  if (n_all == 0) {  // uniform
+    if (wave == 0) store_dims<N, H16>(op, o, 0.f);
     return;
   }
-  const int64_t stride = (int64_t)d.z * kPartRow;  // floats between a head's partials
-  const float* pbase = part + ((int64_t)d.x + hq - cg * kMaxCols) * kPartRow;
+  // this wave's partials: s = wave + WAVES * j, j < ns
+  const int ns = (n_all - wave + WAVES - 1) / WAVES;
+  const int64_t stride = (int64_t)d.z * kPartRow * WAVES;  // floats between them
+  const float* pbase = part + ((int64_t)d.x + hq - cg * kMaxCols) * kPartRow +
+                       (int64_t)d.z * kPartRow * wave;
   const float* po = pbase + N * lane;
-  float2 ml0 = {-INFINITY, 0.f}, ml1 = {-INFINITY, 0.f};
-  if (lane < ns) ml0 = *reinterpret_cast<const float2*>(pbase + lane * stride + D);
-  if (lane + 64 < ns) ml1 = *reinterpret_cast<const float2*>(pbase + (lane + 64) * stride + D);
-  float v0[16][N];
+  float2 ml[kPer];
 #pragma unroll
-  for (int u = 0; u < 16; ++u) {
+  for (int k = 0; k < kPer; ++k) {
+    ml[k] = float2{-INFINITY, 0.f};
+    const int j = lane + 64 * k;
+    if (j < ns) ml[k] = *reinterpret_cast<const float2*>(pbase + j * stride + D);
+  }
+  float v0[kFirst][N];
+#pragma unroll
+  for (int u = 0; u < kFirst; ++u) {
     if (u < ns) {
       load_dims<N>(po + u * stride, v0[u]);
     } else {
@@ -490,35 +514,66 @@ __device__ __forceinline__ void decode_combine(
       for (int i = 0; i < N; ++i) v0[u][i] = 0.f;
     }
   }
-  // lane l holds partials l and l + 64 (ns <= kMaxSlots = 128): the global max and
-  // the weights w_s = 2^(m_s - M) with two wave reductions, then each lane
-  // accumulates its output dims over the partials in order (the first sixteen came
-  // with the (m, l) pairs; the rest in batches of eight loads in flight)
-  const float M = wave_max(fmaxf(ml0.x, ml1.x));
-  const float w0 = (ml0.x == -INFINITY) ? 0.f : fast_exp2(ml0.x - M);
-  const float w1 = (ml1.x == -INFINITY) ? 0.f : fast_exp2(ml1.x - M);
-  const float L = wave_sum(w0 * ml0.y + w1 * ml1.y);
+  // the wave's max and the weights w_s = 2^(m_s - M) with two wave reductions, then each lane
+  // accumulates its output dims over the partials in order (the first came with the
+  // (m, l) pairs; the rest in batches of eight loads in flight)
+  float M = ml[0].x;
 #pragma unroll
-  for (int u = 0; u < 16; ++u) {
-    const float w = __shfl(w0, u, 64);
+  for (int k = 1; k < kPer; ++k) M = fmaxf(M, ml[k].x);
+  M = wave_max(M);
+  float w[kPer], L = 0.f;
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    w[k] = (ml[k].x == -INFINITY) ? 0.f : fast_exp2(ml[k].x - M);
+    L += w[k] * ml[k].y;
+  }
+  L = wave_sum(L);
+#pragma unroll
+  for (int u = 0; u < kFirst; ++u) {
+    const float wu = __shfl(w[0], u, 64);
     if (u < ns) {  // uniform
 #pragma unroll
-      for (int i = 0; i < N; ++i) o[i] = fmaf(w, v0[u][i], o[i]);
+      for (int i = 0; i < N; ++i) o[i] = fmaf(wu, v0[u][i], o[i]);
     }
   }
-  for (int s = 16; s < ns; s += 8) {  // uniform
+  for (int s = kFirst; s < ns; s += 8) {  // uniform
     float v[8][N];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       if (s + u < ns) load_dims<N>(po + (s + u) * stride, v[u]);
     }
+    float wk = w[0];  // uniform select: eight rows never straddle two of a lane's weights
+#pragma unroll
+    for (int k = 1; k < kPer; ++k) wk = s >= 64 * k ? w[k] : wk;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const float w = __shfl(s + u < 64 ? w0 : w1, (s + u) & 63, 64);  // uniform select
+      const float wu = __shfl(wk, (s + u) & 63, 64);
       if (s + u < ns) {
 #pragma unroll
-        for (int i = 0; i < N; ++i) o[i] = fmaf(w, v[u][i], o[i]);
+        for (int i = 0; i < N; ++i) o[i] = fmaf(wu, v[u][i], o[i]);
       }
+    }
+  }
+  if constexpr (WAVES > 1) {
+    __shared__ float so[WAVES][N][64];
+    __shared__ float2 sml[WAVES];
+#pragma unroll
+    for (int i = 0; i < N; ++i) so[wave][i][lane] = o[i];
+    if (lane == 0) sml[wave] = float2{M, L};
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int x = 1; x < WAVES; ++x) M = fmaxf(M, sml[x].x);
+    L = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) o[i] = 0.f;
+#pragma unroll
+    for (int x = 0; x < WAVES; ++x) {
+      const float2 p = sml[x];
+      const float wx = p.x == -INFINITY ? 0.f : fast_exp2(p.x - M);
+      L = fmaf(wx, p.y, L);
+#pragma unroll
+      for (int i = 0; i < N; ++i) o[i] = fmaf(wx, so[x][i][lane], o[i]);
     }
   }
   store_dims<N, H16>(op, o, L > 0.f ? 1.f / L : 0.f);

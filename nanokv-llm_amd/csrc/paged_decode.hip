@@ -69,14 +69,15 @@ void paged_decode_split_kernel(
                                 n_blocks, min_chunks, scale_log2, v_scale, part, desc);
 }
 
-// One wave per (sequence, query head).
-template <int D, bool H16 = false>
-__global__ __launch_bounds__(64) void paged_decode_combine_kernel(
+// One workgroup (of one wave, or four) per (sequence, query head).
+template <int D, bool H16 = false, int WAVES = 1>
+__global__ __launch_bounds__(64 * WAVES) void paged_decode_combine_kernel(
     const int32_t* __restrict__ context_lens, int32_t Hq, int32_t Hk, int32_t NCG,
     const float* __restrict__ part, const i32x4v_t* __restrict__ desc,
     bf16_t* __restrict__ out, int64_t out_row_stride) {
-  decode_combine<D, H16>(DecodeSeqs{context_lens, 0}, (int)blockIdx.x / Hq,
-                         (int)blockIdx.x % Hq, Hq, Hk, NCG, part, desc, out, out_row_stride);
+  decode_combine<D, H16, WAVES>(DecodeSeqs{context_lens, 0}, (int)blockIdx.x / Hq,
+                                (int)blockIdx.x % Hq, Hq, Hk, NCG, part, desc, out,
+                                out_row_stride);
 }
 
 static int decode_check(const void* q, const void* k_cache, const void* v_cache,
@@ -330,14 +331,25 @@ static int decode_combine(const int32_t* context_lens, int32_t batch, int32_t n_
   const i32x4v_t* desc = static_cast<const i32x4v_t*>(workspace);
   const float* part = reinterpret_cast<const float*>(static_cast<const char*>(workspace) + desc_b);
   const dim3 grid((unsigned)(batch * n_q_heads));
-#define NKV_COMBINE_LAUNCH(D)                                                                  \
-  hipLaunchKernelGGL((paged_decode_combine_kernel<D, H16>), grid, dim3(64), 0,                 \
+  // Four waves where a row may have more partials than one wave has loads in flight (16): at
+  // most one for every wave of its head group that the batch leaves to it, and no more than the
+  // table width lets a segment have.
+  const int64_t shares = (int64_t)device_cus() * kWavesPerCU / n_kv_heads / batch + 2;
+  const bool wide = std::min(shares, decode_slots(max_blocks_per_seq, block_size)) > 16;
+#define NKV_COMBINE_LAUNCH_W(D, W)                                                             \
+  hipLaunchKernelGGL((paged_decode_combine_kernel<D, H16, W>), grid, dim3(64 * W), 0,          \
                      as_stream(stream), context_lens, n_q_heads, n_kv_heads, ncg, part, desc,  \
                      (bf16_t*)out, out_row_stride)
+#define NKV_COMBINE_LAUNCH(D)                                                                  \
+  do {                                                                                         \
+    if (wide) NKV_COMBINE_LAUNCH_W(D, 4);                                                      \
+    else NKV_COMBINE_LAUNCH_W(D, 1);                                                           \
+  } while (0)
   if (head_dim == 64) NKV_COMBINE_LAUNCH(64);
   else if (head_dim == 128) NKV_COMBINE_LAUNCH(128);
   else NKV_COMBINE_LAUNCH(256);
 #undef NKV_COMBINE_LAUNCH
+#undef NKV_COMBINE_LAUNCH_W
   return check_launch("nkv_paged_decode_combine");
 }
 }  // namespace nkv

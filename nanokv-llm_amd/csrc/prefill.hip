@@ -852,8 +852,8 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(
     const int id = ((int)blockIdx.x - n_tile_blocks) * kMergeWaves + wave;
     const int b = id / Hq;
     if (b < sa.n_seqs && cu_q[b + 1] - cu_q[b] == 1)  // uniform over the wave
-      decode_combine<D, H16>(OneRowSeqs{cu_q, cu_k, sa.n_seqs}, b, id - b * Hq, Hq, Hk, sa.ncg,
-                             sa.row_part, sa.row_desc, out, out_row_stride);
+      decode_combine<D, H16, 1>(OneRowSeqs{cu_q, cu_k, sa.n_seqs}, b, id - b * Hq, Hq, Hk,
+                                sa.ncg, sa.row_part, sa.row_desc, out, out_row_stride);
     return;
   }
   const int x = blockIdx.x % n_groups;
