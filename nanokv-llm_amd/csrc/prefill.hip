@@ -112,18 +112,27 @@ struct SplitArgs {
   i32x4v_t* row_desc;
   float* row_part;
 };
-constexpr int kMinRange = 20;  // cost units (four key steps of a full tile)
 constexpr int kSnap = 2;  // a range never cuts a unit within this many steps of its ends
 
 // Floats of a partial row: O, m, l, 2 pad.
 constexpr int prefill_part_row(int D) { return D + 4; }
 
-// Cost of one key step of a tile with `rows` rows: the tile's K/V bytes plus a share for
-// each wave that has rows to compute.
+// Cost of one key step of a tile with `rows` rows: its loads and the step's latency, and a share
+// for each wave that has rows to compute. With a smaller base (1 of 5) a range of a sequence's
+// last, partial tile took up to twice the others' time: 1522 tokens in two chunks on 9000 (Hq 16,
+// Hk 8) 207 us, with 5 of 9 155; three chunks and 10 decode rows 70.5, 65.1.
+constexpr int kStepBase = 5;
+constexpr int kFullStep = kStepBase + 4;
+constexpr int kMinRange = 4 * kFullStep;
+// Shortest range over all heads' T tile steps: sqrt(T) / 6 steps. A range's part costs about 7
+// steps to write and merge (100 KB each way), so halving the ranges of a small call gains until
+// its steps take as long: four chunks of 75 - 195 tokens on 2650 (Hq 16, Hk 2) 52.5 -> 46.4 us;
+// no range of a call that fills the chip is touched.
+constexpr float kRangeRoot = 1.f / 6.f;
 template <int D, bool F8>
 __device__ __forceinline__ int step_cost(int rows) {
   constexpr int kWaveRows = 16 * prefill_row_groups(D, F8);
-  return 1 + (rows + kWaveRows - 1) / kWaveRows;
+  return kStepBase + (rows + kWaveRows - 1) / kWaveRows;
 }
 // Key steps of tile t (at least one, which an empty tile masks whole).
 __device__ __forceinline__ int tile_steps(int Lq, int Lk, int qt, int t) {
@@ -136,7 +145,7 @@ __device__ __forceinline__ int tile_steps(int Lq, int Lk, int qt, int t) {
 // stream them as the decode kernel does, bound by the K/V bytes, beside the workgroups that
 // the prompts' tiles keep at the matrix cores. A 192-row tile for one row ran at 5.2 TB/s of
 // K/V (a 256-byte piece of each row and 64 keys in flight a workgroup; decode_stream: 6.5).
-// Cost of a 16-key chunk of one head, in quarters of a tile step's units: fewer workgroups than
+// Cost of a 16-key chunk of one head, in twentieths of a full tile's step: fewer workgroups than
 // their share of the time alone would give them (5 and 3), since the memory serves the rows
 // at its full rate from half the chip's waves while the others compute. 48 rows with two
 // 512-token chunks, at 1, 2, 3, 4, 6: 116, 117, 126, 129, 160 us; 80 rows of 4k - 8k with one:
@@ -188,7 +197,7 @@ __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
   int n_ranges = (int)gridDim.x / Hk;  // of each KV head
   c.row_groups = 0;
   if constexpr (ROWS) {  // shared out by cost, at least a range of each kind that there is
-    const int rows = __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63) * row_cost(F8) / 4;
+    const int rows = __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63) * row_cost(F8) * kFullStep / 20;
     if (rows > 0) {
       const int r = (int)((float)n_ranges * (float)rows / (float)(rows + T) + 0.5f);
       const int r_rows = T > 0 ? min(max(r, 1), n_ranges - 1) : n_ranges;
@@ -198,7 +207,9 @@ __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
     if ((int)blockIdx.x < c.row_groups) return false;
   }
   c.group = (int)blockIdx.x - c.row_groups;
-  c.C = max((T + n_ranges - 1) / max(n_ranges, 1), sa.min_range);
+  const float steps = (float)T * (float)Hk / kFullStep;
+  c.C = max(max((T + n_ranges - 1) / max(n_ranges, 1), sa.min_range),
+            (int)(sqrtf(steps) * (kRangeRoot * kFullStep)));
   const int x = c.group / Hk * c.C;
   if (x >= T) return false;
   c.x = x;
