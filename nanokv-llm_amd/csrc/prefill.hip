@@ -10,10 +10,11 @@
 //    The tile's R "rows" are its queries for all g query heads of the KV
 //    head, query-major (row r = query r/g, head r%g; rows past the tile's
 //    queries x g are computed and dropped), so one K/V tile in LDS serves g
-//    heads (GQA sharing). Wave w owns three 16-row groups at head_dim 128
+//    heads (GQA sharing). Wave w owns up to three 16-row groups at head_dim 128
 //    (R = 192), two at 64 and in the fp8 instance (R = 128), one at 256
-//    (R = 64, and the 128 KiB ring leaves one workgroup per CU). head_dim D
-//    is 64, 128 or 256 (a template parameter).
+//    (R = 64, and the 128 KiB ring leaves one workgroup per CU); fewer where
+//    the batch has few tiles (prefill_groups). head_dim D is 64, 128 or 256 (a
+//    template parameter).
 //  * Keys advance in 64-key steps. Each step's K and V tiles (2 x 16 KiB at
 //    D = 128) go from HBM straight into LDS with gfx950's 16-byte buffer-load-to-LDS
 //    (no staging registers, no LDS write instructions) through a ring of
@@ -52,14 +53,14 @@ namespace nkv {
 constexpr int kStep = 64;                 // keys per step
 constexpr int kStages = 2;                // LDS ring depth (steps)
 constexpr bool prefill_dim_ok(int D) { return D == 64 || D == 128 || D == 256; }
-// 16-row groups per wave: three at head_dim 128 (each K and V^T read from LDS serves three
+// Most 16-row groups per wave: three at head_dim 128 (each K and V^T read from LDS serves three
 // MFMAs; bit-identical to two, at par to 2% faster), two at 64 and in the fp8 instance (whose
 // staging registers leave no room for a third), one at 256 (its O^T and Q^T registers
 // would not fit two waves per SIMD otherwise)
 constexpr int prefill_row_groups(int D, bool F8) {
   return D == 256 ? 1 : (D == 128 && !F8 ? 3 : 2);
 }
-// rows (query, head pairs) of a workgroup's tile: 4 waves
+// rows (query, head pairs) of the largest tile, the split launch's: 4 waves
 constexpr int prefill_tile_rows(int D, bool F8) { return 64 * prefill_row_groups(D, F8); }
 // largest GQA group, the same for every instance of a head_dim: each tile holds at least
 // one query for all g heads of its KV head
@@ -197,7 +198,8 @@ __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
   int n_ranges = (int)gridDim.x / Hk;  // of each KV head
   c.row_groups = 0;
   if constexpr (ROWS) {  // shared out by cost, at least a range of each kind that there is
-    const int rows = __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63) * row_cost(F8) * kFullStep / 20;
+    const int rows =
+        __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63) * row_cost(F8) * kFullStep / 20;
     if (rows > 0) {
       const int r = (int)((float)n_ranges * (float)rows / (float)(rows + T) + 0.5f);
       const int r_rows = T > 0 ? min(max(r, 1), n_ranges - 1) : n_ranges;
@@ -262,7 +264,7 @@ __device__ __forceinline__ bool split_next(const int32_t* __restrict__ cu_q,
 // units, each unit's key steps [s_lo, s_end) of n_steps (SPLIT).
 // HP (SPLIT, paged): KV heads a wave of the decode rows reads at once, 0 for decode rows as
 // tiles of one query.
-template <bool F8, int D, bool H16, bool PAGED, bool SPLIT, int HP = 0>
+template <bool F8, int D, bool H16, bool PAGED, int RG, bool SPLIT, int HP = 0>
 __device__ __forceinline__ void prefill_body(
     const bf16_t* __restrict__ q, int64_t q_row_stride, const void* __restrict__ k_cache,
     const void* __restrict__ v_cache, int64_t k_row_stride, int64_t v_row_stride,
@@ -275,7 +277,7 @@ __device__ __forceinline__ void prefill_body(
   constexpr int kEl = F8 ? 1 : 2;          // bytes per cache element
   constexpr int kRB = D * 2;               // bytes of a staged (bf16) K or V row
   constexpr int kNC = D / 8;               // 16-byte chunks per staged row
-  constexpr int kRG = prefill_row_groups(D, F8);
+  constexpr int kRG = RG;
   constexpr int kTileB = kStep * kRB;      // bytes of one K or V tile
   constexpr int kStageB = 2 * kTileB;      // K tile then V tile
   constexpr int kKs = D / 32;              // k-steps of S^T
@@ -285,7 +287,7 @@ __device__ __forceinline__ void prefill_body(
   constexpr int kLpr8 = D / 16;            // F8: lanes per row (16 codes each)
   constexpr int kRpl8 = 64 / kLpr8;        // F8: rows per load
   constexpr int kNl8 = 16 / kRpl8;         // F8: loads per wave per tile
-  const int QT = prefill_tile_rows(D, F8) / G;  // queries per tile
+  const int QT = 64 * RG / G;  // queries per tile
   constexpr int kRowLds = 2 * decode_lds_elems<F8, HP == 0 ? 1 : HP, D>();  // bytes a wave
   constexpr int kRingB = kStages * kStageB;
   __shared__ __attribute__((aligned(1024))) char
@@ -372,7 +374,7 @@ __device__ __forceinline__ void prefill_body(
   // workgroup describes the unit to the merge.
   auto part_tile = [&]() {
     return sa.part + ((int64_t)blockIdx.x * 2 + (s_lo == 0)) *
-                         (prefill_tile_rows(D, F8) * prefill_part_row(D));
+                         (64 * RG * prefill_part_row(D));
   };
   auto describe = [&]() {
     const int w0 = (cur.u0 + snap + cur.C - 1) / cur.C;  // the unit's first cut
@@ -826,24 +828,24 @@ __device__ __forceinline__ void prefill_body(
       block_tables, bt_row_stride, Hk, G, block_size, max_blocks, n_limit, n_tiles, scale_log2, \
       v_scale, out, out_row_stride
 
-template <bool F8, int D, bool H16, bool PAGED>
+template <bool F8, int D, bool H16, bool PAGED, int RG>
 __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void prefill_varlen_kernel(
     NKV_PREFILL_PARAMS) {
-  prefill_body<F8, D, H16, PAGED, false>(NKV_PREFILL_PASS, SplitArgs{});
+  prefill_body<F8, D, H16, PAGED, RG, false>(NKV_PREFILL_PASS, SplitArgs{});
 }
 
 template <bool F8, int D, bool H16, bool PAGED, int HP>
 __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void prefill_split_kernel(
     NKV_PREFILL_PARAMS, const SplitArgs sa) {
-  prefill_body<F8, D, H16, PAGED, true, HP>(NKV_PREFILL_PASS, sa);
+  prefill_body<F8, D, H16, PAGED, prefill_row_groups(D, F8), true, HP>(NKV_PREFILL_PASS, sa);
 }
 
 // Merges the parts of the units that ranges cut: descriptor x (of the workgroup that holds a
 // unit's first part; part p > 0 is in the first slot of the workgroup p * Hk after it) and rows
 // 32*y .. of its tile (block y * groups + x). The blocks after those merge the decode rows'
-// partials, one (sequence, query head) a wave. A wave merges four rows at once, lane l output dims N*l .. N*l+N-1, eight
-// parts' loads in flight. Where the rows leave waves idle (a decode row's tile has G) they take
-// every n-th part each and merge once more through LDS.
+// partials, one (sequence, query head) a wave. A wave merges four rows at once, lane l output
+// dims N*l .. N*l+N-1, eight parts' loads in flight. Where the rows leave waves idle (a decode
+// row's tile has G) they take every n-th part each and merge once more through LDS.
 constexpr int kMergeRows = 32;
 constexpr int kMergeWaves = kMergeRows / 4;
 template <int D, bool H16>
@@ -993,19 +995,65 @@ static int prefill_row_heads(int32_t n_kv_heads, int32_t G, int32_t head_dim) {
   return 1;
 }
 
-// Whether the split launch is the faster one, from what the host knows: the longest lengths, the
-// rows of q and how many sequences share them (with as few prompts as could bring them, the
-// others being decode rows). In us, on times fitted to both sides of 130 random steps (1 - 104
-// sequences, 1 - 3000 new tokens, contexts of up to 16k, every KV type):
-//  * plain, the workgroup of the longest sequence's last tile walks its keys alone, 1.7 a 64-key
-//    step, however few tiles there are; with many decode rows each takes a tile's time, 6 a step
-//    for as many as the chip holds;
-//  * split, every workgroup has an equal share: 2.8 a step of the tiles and 1 of the rows (their
-//    bytes), and 35 for the launch, the parts' writing and the merge.
+// What the host knows of a batch's composition: as few prompts as could bring its rows of q
+// (total_q; every sequence's max_seqlen_q where it is not known), the others being decode rows.
+struct BatchMix {
+  int64_t prompts, rows, prompt_rows;  // prompts, decode rows, the prompts' rows of q
+};
+static BatchMix batch_mix(int64_t n_seqs, int64_t total_q, int64_t max_seqlen_q) {
+  if (total_q < 0) total_q = n_seqs * max_seqlen_q;
+  const int64_t more = std::max<int64_t>(0, total_q - n_seqs);  // beyond one token each
+  BatchMix m;
+  m.prompts = max_seqlen_q > 1
+                  ? std::min(n_seqs, (more + max_seqlen_q - 2) / (max_seqlen_q - 1))
+                  : 0;
+  m.rows = n_seqs - m.prompts;
+  m.prompt_rows = total_q - m.rows;
+  return m;
+}
+
+// Row groups per wave of a plain launch (every number gives the same bits). More rows a tile
+// need fewer reads of K and V from LDS per MFMA, fewer leave more workgroups to overlap, and a
+// workgroup's key step takes 1.15 us with one, 1.26 with two, 1.75 with three while the chip is
+// not full. Measured (Hq 32, Hk 8; 1 / 2 / 3 groups, us; workgroups as with three):
+//   a prompt of 333 (56 workgroups)     11.2 /  14.4 /  20.2
+//   of 1500 (256)                       33.4 /  38.0 /  51.6
+//   of 3000 (504)                       95.5 /  80.2 /  98.3
+//   four chunks of 2048 on 6000 (1376)  1053 /   809 /   841
+//   16 prompts up to 1500 (3144)         305 /   229 /   241
+//   16 prompts up to 4096 (8472)        1682 /  1315 /  1294
+//   80 decode rows, a prompt of 300      34.3 /  51.0 /  46.9 (a row's tile is a row)
+static int prefill_groups(int64_t n_seqs, int64_t total_q, int64_t max_seqlen_q,
+                          int32_t n_kv_heads, int g, int32_t head_dim, bool f8) {
+  const int most = prefill_row_groups(head_dim, f8);
+  const BatchMix m = batch_mix(n_seqs, total_q, max_seqlen_q);
+  const int64_t qt = 64 * most / g;
+  const int64_t tiles =
+      std::min(m.prompts * ((max_seqlen_q + qt - 1) / qt), m.prompt_rows / qt + m.prompts);
+  const int64_t groups = (tiles + m.rows) * n_kv_heads;
+  const int64_t cus = device_cus();
+  const int want = g <= 64 && (groups <= cus || m.rows >= tiles) ? 1
+                   : groups <= 16 * cus                          ? std::min(most, 2)
+                                                                 : most;
+  // every sequence's tiles are launched as for the longest: more of them only while the empty
+  // ones are few, and no launch grows past what the largest tiles would take beyond that
+  const int64_t q = 64 * want / g;
+  return n_seqs * ((max_seqlen_q + q - 1) / q) * n_kv_heads <= (1 << 16) ? want : most;
+}
+
+// Whether the split launch is the faster one, from what the host knows of the lengths and the
+// batch's mix. In us, fitted to both sides' times of 200 random steps (1 - 104 sequences, 1 -
+// 3000 new tokens, contexts of up to 16k, every KV type):
+//  * plain, the workgroup of the longest sequence's last tile walks its keys alone, 1.0 a 64-key
+//    step with the small tiles of a few workgroups; else every step of a tile costs its share
+//    of the chip, 1.5, and of a decode row 4;
+//  * split, the tiles' steps cost the same, the rows' (their bytes) 0.25, and the launch, the
+//    parts' writing and the merge 35.
 // The keys of a batch are taken as half of the longest sequence's. The rule's choice was at most
-// 7% slower than the plain launch (one step of 130), up to 4.9x faster, and lost 0.7% against
-// always knowing the faster. 512 tokens on 12288 (Hq 32, Hk 8): 338 -> 138 us; 48 decode rows
-// with two 512-token chunks: 208 -> 117 us.
+// 16% slower than the plain launch (five steps of 200 over 10%), up to 3.0x faster, and lost
+// 1.2% against always knowing the faster. One layer's call of 512 tokens on 12288 (Hq 32,
+// Hk 8): 181 us plain (347 with 192-row tiles), 133 split; of 48 decode rows with two 512-token
+// chunks: 237 and 123.
 static bool prefill_split_wins(int32_t n_seqs, int64_t total_q, int32_t max_seqlen_q,
                                int32_t max_seqlen_k, int32_t n_q_heads, int32_t n_kv_heads,
                                int32_t head_dim, bool f8) {
@@ -1015,12 +1063,9 @@ static bool prefill_split_wins(int32_t n_seqs, int64_t total_q, int32_t max_seql
   // every range counts the tiles of the sequences before it: not for long prompts (whose
   // tiles fill the chip anyway)
   if (tiles_max > 96 || max_seqlen_k < max_seqlen_q) return false;
-  const int64_t more = std::max<int64_t>(0, total_q - n_seqs);  // beyond one token each
-  const int64_t prompts =
-      max_seqlen_q > 1 ? std::min<int64_t>(n_seqs, (more + max_seqlen_q - 2) / (max_seqlen_q - 1))
-                       : 0;
-  const int64_t rows = n_seqs - prompts;
-  const int64_t tiles = std::min(prompts * tiles_max, (total_q - rows) / qt + prompts);
+  const BatchMix m = batch_mix(n_seqs, total_q, max_seqlen_q);
+  const int64_t tiles = std::min(m.prompts * tiles_max, m.prompt_rows / qt + m.prompts);
+  const int64_t rows = m.rows;
   const double steps = (max_seqlen_k + kStep - 1) / kStep;
   // positions of the stream are 32 bits
   if ((tiles + rows) * steps * 8 >= 2147483648.0) return false;
@@ -1029,8 +1074,8 @@ static bool prefill_split_wins(int32_t n_seqs, int64_t total_q, int32_t max_seql
   const double tile_steps = tiles * steps * seen * per_range * (n_seqs == 1 ? 1.0 : 0.5);
   const double row_steps = rows * steps * 0.5 * per_range;
   const double dim = head_dim / 128.0;
-  return dim * std::max(1.7 * steps, 2.5 * tile_steps + 6.0 * row_steps) >
-         35.0 + dim * (2.8 * tile_steps + row_steps);
+  return dim * std::max(steps, 1.5 * tile_steps + 4.0 * row_steps) >
+         35.0 + dim * (1.5 * tile_steps + 0.25 * row_steps);
 }
 
 // `split`: a split launch over `workspace`; a plain one otherwise.
@@ -1043,7 +1088,7 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
                           int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim,
                           int32_t block_size, int64_t n_rows, float scale, float k_scale,
                           float v_scale, void* out, int64_t out_row_stride, void* stream,
-                          bool split = false, void* workspace = nullptr,
+                          int64_t total_q = -1, bool split = false, void* workspace = nullptr,
                           size_t workspace_bytes = 0) {
   constexpr int kEl = F8 ? 1 : 2;
   const char* what = F8 ? "prefill_varlen_fp8" : H16 ? "prefill_varlen_f16" : "prefill_varlen";
@@ -1087,7 +1132,10 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
   // paged: valid block ids are [0, n_rows / block_size); contiguous: valid rows
   const int32_t n_limit = (int32_t)std::min<int64_t>(block_tables ? n_rows / block_size : n_rows,
                                                      INT32_MAX);
-  const int tile_rows = prefill_tile_rows(head_dim, F8);
+  const int groups = split ? prefill_row_groups(head_dim, F8)
+                           : prefill_groups(n_seqs, total_q, max_seqlen_q, n_kv_heads, g,
+                                            head_dim, F8);
+  const int tile_rows = 64 * groups;
   const int qt = tile_rows / g;
   const int n_tiles = (max_seqlen_q + qt - 1) / qt;
   const float sl2 = scale * k_scale * kLog2e;
@@ -1127,14 +1175,18 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
   (const bf16_t*)q, q_row_stride, k_cache, v_cache, k_row_stride, v_row_stride, cu_seqlens_q,  \
       cu_seqlens_k, block_tables, bt_row_stride, n_kv_heads, g, block_size, max_blocks,        \
       n_limit, n_tiles, sl2, v_scale, (bf16_t*)out, out_row_stride
+#define NKV_PREFILL_PLAIN(D, P, RG)                                                            \
+  hipLaunchKernelGGL((prefill_varlen_kernel<F8, D, H16, P, RG>), dim3((unsigned)grid),         \
+                     dim3(256), 0, as_stream(stream), NKV_PREFILL_ARGS)
 #define NKV_PREFILL_SPLIT(D, P, HP)                                                            \
   hipLaunchKernelGGL((prefill_split_kernel<F8, D, H16, P, HP>), dim3((unsigned)grid), dim3(256), \
                      0, as_stream(stream), NKV_PREFILL_ARGS, sa)
 #define NKV_PREFILL_LAUNCH_P(D, P)                                                             \
   do {                                                                                         \
     if (!split) {                                                                              \
-      hipLaunchKernelGGL((prefill_varlen_kernel<F8, D, H16, P>), dim3((unsigned)grid),         \
-                         dim3(256), 0, as_stream(stream), NKV_PREFILL_ARGS);                   \
+      if (groups == 1) NKV_PREFILL_PLAIN(D, P, 1);                                             \
+      else if (groups == 2) NKV_PREFILL_PLAIN(D, P, std::min(2, prefill_row_groups(D, F8)));   \
+      else NKV_PREFILL_PLAIN(D, P, prefill_row_groups(D, F8));                                 \
       break;                                                                                   \
     }                                                                                          \
     if constexpr (P) {                                                                         \
@@ -1166,10 +1218,33 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
   else NKV_PREFILL_LAUNCH(256);
 #undef NKV_PREFILL_LAUNCH
 #undef NKV_PREFILL_LAUNCH_P
+#undef NKV_PREFILL_PLAIN
 #undef NKV_PREFILL_SPLIT
 #undef NKV_PREFILL_ARGS
   return check_launch(F8 ? "nkv_prefill_varlen_fp8"
                          : H16 ? "nkv_prefill_varlen_f16" : "nkv_prefill_varlen");
+}
+}  // namespace nkv
+
+namespace nkv {
+int prefill_plain(int32_t kv_type, const void* q, int64_t q_row_stride, const void* k_cache,
+                  const void* v_cache, int64_t row_stride, const int32_t* cu_seqlens_q,
+                  const int32_t* cu_seqlens_k, const int32_t* block_tables,
+                  int64_t bt_row_stride, int32_t max_blocks_per_seq, int32_t n_seqs,
+                  int64_t total_q, int32_t max_seqlen_q, int32_t n_q_heads, int32_t n_kv_heads,
+                  int32_t head_dim, int32_t block_size, int64_t n_rows, float scale,
+                  float k_scale, float v_scale, void* out, int64_t out_row_stride,
+                  void* stream) {
+#define NKV_PREFILL_ANY(...)                                                                   \
+  prefill_launch<__VA_ARGS__>(q, q_row_stride, k_cache, v_cache, row_stride, row_stride,       \
+                              cu_seqlens_q, cu_seqlens_k, block_tables, bt_row_stride,         \
+                              max_blocks_per_seq, n_seqs, max_seqlen_q, n_q_heads, n_kv_heads, \
+                              head_dim, block_size, n_rows, scale, k_scale, v_scale, out,      \
+                              out_row_stride, stream, total_q)
+  if (kv_type == NKV_KV_FP8) return NKV_PREFILL_ANY(true);
+  if (kv_type == NKV_KV_F16) return NKV_PREFILL_ANY(false, true);
+  return NKV_PREFILL_ANY(false);
+#undef NKV_PREFILL_ANY
 }
 }  // namespace nkv
 
@@ -1273,7 +1348,7 @@ extern "C" int nkv_prefill_varlen_split(int32_t kv_type, const void* q, int64_t 
                               cu_seqlens_q, cu_seqlens_k, block_tables, bt_row_stride,         \
                               max_blocks_per_seq, n_seqs, max_seqlen_q, n_q_heads, n_kv_heads, \
                               head_dim, block_size, n_rows, scale, k_scale, v_scale, out,      \
-                              out_row_stride, stream, true, workspace, workspace_bytes)
+                              out_row_stride, stream, -1, true, workspace, workspace_bytes)
   switch (kv_type) {
     case NKV_KV_BF16: return NKV_PREFILL_SPLIT(false);
     case NKV_KV_F16: return NKV_PREFILL_SPLIT(false, true);

@@ -158,6 +158,30 @@ def test_attention_takes_a_long_prefix_to_the_split_launch(nkv, dev):
     nkv.reset_context()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,Hq,Hk,D", [("bf16", 32, 8, 128), ("fp16", 20, 4, 128),
+                                          ("fp8", 16, 2, 128), ("bf16", 8, 2, 64),
+                                          ("bf16", 128, 1, 128)])
+@pytest.mark.parametrize("n", [1, 30, 70])
+def test_plain_tile_sizes_match_the_oracle(nkv, dev, kind, Hq, Hk, D, n):
+    """Plain launches of one, two and three row groups a wave: the first sequences' lengths stand
+    at the edges of their tiles, the others fill up to the workgroups that change the size."""
+    g = Hq // Hk
+    mix = [(max(1, 64 * rg // g + d), 70 * rg + d) for rg in (1, 2, 3) for d in (-1, 0, 1)]
+    mix = [(min(a, b), b) for a, b in mix][:9] + [(400, 400)] * (n > 1) + [(250, 300)] * (n - 1)
+    q, k, v, cu_q, cu_k, bt = _inputs(dev, mix, Hq, Hk, D, kind, 64, True, seed=11)
+    s = 1 / 16 if kind == "fp8" else 1.0
+    out = nkv.varlen_prefill(*(x.to(dev) for x in (q, k, v, cu_q, cu_k)),
+                             max(a for a, _ in mix), D ** -0.5, block_tables=bt.to(dev),
+                             k_scale=s, v_scale=s)
+    torch.cuda.synchronize()
+    some = 10  # sequences compared
+    ref = varlen_prefill_ref(q[:int(cu_q[some - 1])].float(), k.float() * s, v.float() * s,
+                             cu_q[:some], cu_k[:some], D ** -0.5, block_tables=bt[:some - 1])
+    assert (out[:ref.size(0)].float().cpu() - ref).abs().max().item() <= TOL
+    assert bool(torch.isfinite(out.float()).all())
+
+
 def test_split_plan_and_arguments_on_the_host():
     """The rule, and what the entry point refuses, without a GPU."""
     lib = L.lib()
