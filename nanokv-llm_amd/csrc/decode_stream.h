@@ -11,7 +11,7 @@
 namespace nkv {
 
 constexpr int kChunk = 16;               // tokens per pipeline stage
-constexpr int kMinChunks = 4;            // minimum chunks per wave range
+constexpr int kMinChunks = 4;            // chunks per wave range that grids are sized for
 // partials per (sequence, query head) at most: what four waves' combine has in flight at once
 // (4 x 32), and one, so that a table of 512 chunks splits into ranges of 4
 constexpr int kMaxSlots = 129;
@@ -32,22 +32,27 @@ typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
 typedef __bf16 bf16x2v_t __attribute__((ext_vector_type(2)));
 typedef int32_t i32x4v_t __attribute__((ext_vector_type(4)));
 
-// Partial slots per (sequence, query head): a segment of n chunks is touched by at most
-// ceil(n / C) + 1 waves, and the kernel takes C >= decode_min_chunks, which is at least
-// kMinChunks and at least max_chunks / (slots - 1), so no segment has more than kMaxSlots
-// partials (as many as the combine holds).
-static inline int64_t decode_slots(int32_t max_blocks, int32_t block_size) {
-  const int64_t max_chunks = ((int64_t)max_blocks * block_size + kChunk - 1) / kChunk;
-  const int64_t s = (max_chunks + kMinChunks - 1) / kMinChunks + 1;
-  return s < kMaxSlots ? s : kMaxSlots;
+static inline int64_t decode_max_chunks(int32_t max_blocks, int32_t block_size) {
+  return ((int64_t)max_blocks * block_size + kChunk - 1) / kChunk;
 }
-// The smallest range a wave takes: kMinChunks, or longer when the table width allows
-// segments that would otherwise need more than `slots` partials.
-static inline int32_t decode_min_chunks(int32_t max_blocks, int32_t block_size) {
-  const int64_t max_chunks = ((int64_t)max_blocks * block_size + kChunk - 1) / kChunk;
-  const int64_t slots = decode_slots(max_blocks, block_size);
-  const int64_t c = (max_chunks + slots - 2) / (slots - 1);
-  return (int32_t)(c > kMinChunks ? c : kMinChunks);
+// The smallest range a wave takes. The grid and the workspace are sized for ranges of kMinChunks
+// of full tables; contexts shorter than the table leave some of those waves idle, and shorter
+// ranges use them. A range starts with its first ring slots in flight at once, two chunks of
+// 256-byte row pieces: longer ranges add round trips, shorter ones partials to merge. Measured
+// with 4 / 3 (split and combine in a graph, us): four sequences of 300-1000 12.8 / 11.2, eight
+// 13.8 / 12.4, 24 of 50-250 13.1 / 11.4, 40 of 20-64 12.4 / 10.6, 100 of 50-500 17.9 / 17.1; one
+// or two, whose table fits, gain nothing (11.0 / 11.4). Ranges of two are slower from three
+// sequences on (16 of 100-900, 40 query heads: 13.8 / 15.0). fp8 and head_dim 64 hold four
+// chunks and keep ranges of four.
+static inline int32_t decode_range_floor(int32_t batch, int32_t D, bool f8) {
+  return D == 128 && !f8 && batch > 2 ? 3 : kMinChunks;
+}
+// The smallest range: the floor, or longer where the table width allows segments that would
+// otherwise have more than kMaxSlots partials (a segment of n chunks is touched by at most
+// ceil(n / C) + 1 waves), which is as many as the combine holds.
+static inline int32_t decode_min_chunks(int64_t max_chunks, int32_t floor) {
+  const int64_t c = (max_chunks + kMaxSlots - 2) / (kMaxSlots - 1);
+  return (int32_t)(c > floor ? c : floor);
 }
 
 // Cursor over sequences in batches of 64 (one per lane): in the chunk stream
@@ -235,7 +240,8 @@ __device__ __forceinline__ void decode_stream(
       cur.cb += 64;
       seq_load(cur, seqs, max_tokens);
     }
-    const int ln = __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(cur.base + cur.incl > k)));
+    const int ln =
+        __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(cur.base + cur.incl > k)));
     const int b = cur.cb + ln;
     const int ctx = __builtin_amdgcn_readlane(cur.ctx, ln);
     const int nc = __builtin_amdgcn_readlane(cur.nc, ln);
@@ -460,7 +466,7 @@ __device__ __forceinline__ void decode_stream(
 // sum_s 2^(m_s-M) l_s. Lane l owns output dims N*l .. N*l+N-1. WAVES = 1: the calling wave
 // alone. WAVES > 1: the waves of a workgroup share the partials, wave w those with
 // s % WAVES == w (in its lane s / WAVES), and merge once more through LDS: a context that many
-// waves shared has up to kMaxSlots, and one wave took 10.3 us over the 120 of a 23001-token sequence
+// waves shared has up to kMaxSlots, and one wave took 10.3 us over a 23001-token sequence's 120
 // (a round trip for every eight rows), four waves with 32 rows in flight each 4.2 us.
 template <int D, bool H16, int WAVES, typename Seqs>
 __device__ __forceinline__ void decode_combine(

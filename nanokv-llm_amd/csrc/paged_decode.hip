@@ -168,9 +168,11 @@ struct DecodePlan {
   int32_t min_chunks;
 };
 
+// Waves per head group that full tables give ranges of kMinChunks (or more, see
+// decode_min_chunks).
 static int64_t decode_useful_waves(int32_t batch, int32_t max_blocks, int32_t block_size) {
-  const int64_t max_chunks = ((int64_t)max_blocks * block_size + kChunk - 1) / kChunk;
-  const int32_t min_chunks = decode_min_chunks(max_blocks, block_size);
+  const int64_t max_chunks = decode_max_chunks(max_blocks, block_size);
+  const int32_t min_chunks = decode_min_chunks(max_chunks, kMinChunks);
   return std::max<int64_t>(1, (batch * max_chunks + min_chunks - 1) / min_chunks);
 }
 
@@ -178,7 +180,7 @@ template <bool F8>
 static DecodePlan decode_plan(int32_t batch, int32_t Hq, int32_t Hk, int32_t max_blocks,
                               int32_t block_size, int32_t D) {
   const int g = Hq / Hk;
-  const int64_t max_chunks = ((int64_t)max_blocks * block_size + kChunk - 1) / kChunk;
+  const int64_t max_chunks = decode_max_chunks(max_blocks, block_size);
   // Several KV heads per wave (up to a 512-byte piece of every token row) when the heads
   // group evenly, the hp*G query heads fit the 16 MFMA columns and there is enough work
   // for every wave (upper bound from the table width: >= 32 chunks per head group per
@@ -193,14 +195,14 @@ static DecodePlan decode_plan(int32_t batch, int32_t Hq, int32_t Hk, int32_t max
   DecodePlan p;
   p.hp = hp;
   p.ncg = decode_ncg(g);
-  p.min_chunks = decode_min_chunks(max_blocks, block_size);
+  p.min_chunks = decode_min_chunks(max_chunks, decode_range_floor(batch, D, F8));
   // Resident waves per head group, but no more than the table width lets receive a range
-  // of min_chunks (small batches launch only the waves that can get work).
+  // of kMinChunks (small batches launch only the waves that can get work).
   const int resident = decode_grid_of<F8>(hp, D);
   const int np = Hk * p.ncg / p.hp;
   const int64_t per =
-      std::min<int64_t>(std::max(1, resident / np), decode_useful_waves(batch, max_blocks,
-                                                                        block_size));
+      std::min<int64_t>(std::max(1, resident / np),
+                        decode_useful_waves(batch, max_blocks, block_size));
   p.grid = (unsigned)(per * np);
   return p;
 }
@@ -333,9 +335,12 @@ static int decode_combine(const int32_t* context_lens, int32_t batch, int32_t n_
   const dim3 grid((unsigned)(batch * n_q_heads));
   // Four waves where a row may have more partials than one wave has loads in flight (16): at
   // most one for every wave of its head group that the batch leaves to it, and no more than the
-  // table width lets a segment have.
+  // table width lets a segment have (of a 16-bit pool: an fp8 one's ranges are no shorter).
+  const int64_t max_chunks = decode_max_chunks(max_blocks_per_seq, block_size);
+  const int64_t min_chunks =
+      decode_min_chunks(max_chunks, decode_range_floor(batch, head_dim, false));
   const int64_t shares = (int64_t)device_cus() * kWavesPerCU / n_kv_heads / batch + 2;
-  const bool wide = std::min(shares, decode_slots(max_blocks_per_seq, block_size)) > 16;
+  const bool wide = std::min(shares, (max_chunks + min_chunks - 1) / min_chunks + 1) > 16;
 #define NKV_COMBINE_LAUNCH_W(D, W)                                                             \
   hipLaunchKernelGGL((paged_decode_combine_kernel<D, H16, W>), grid, dim3(64 * W), 0,          \
                      as_stream(stream), context_lens, n_q_heads, n_kv_heads, ncg, part, desc,  \

@@ -1158,7 +1158,9 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
     sa.row_desc = reinterpret_cast<i32x4v_t*>(ws + z.desc + z.part);
     sa.row_part = reinterpret_cast<float*>(ws + z.desc + z.part + z.row_desc);
     sa.ncg = decode_ncg(g);
-    sa.min_chunks = block_tables ? decode_min_chunks(max_blocks, block_size) : 0;
+    sa.min_chunks = block_tables ? decode_min_chunks(decode_max_chunks(max_blocks, block_size),
+                                                     kMinChunks)
+                                 : 0;
     // a range for each kind of work, dense cache rows, and positions of the decode rows' chunks
     // in 32 bits
     if (block_tables && prefill_ranges(n_kv_heads, head_dim) >= 2 &&

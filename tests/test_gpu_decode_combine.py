@@ -38,6 +38,29 @@ def test_merge_of_many_partials(nkv, dev, ctx, D, kind):
     assert (out.float().cpu()[some] - ref).abs().max().item() <= 2e-2
 
 
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "fp8"])
+@pytest.mark.parametrize("B,width", [(16, 4), (16, 5), (256, 2), (256, 16), (256, 17)])
+@pytest.mark.parametrize("batch", [1, 2, 3, 11])
+def test_small_batches_in_short_ranges(nkv, dev, batch, B, width, kind):
+    """Ranges of three and four chunks: batches and table widths around the changes, and
+    contexts that end at and beside a range's end."""
+    g = torch.Generator().manual_seed(batch * width)
+    Hq, Hk, D = 8, 2, 128
+    dt = torch.float16 if kind == "fp16" else torch.bfloat16
+    top = B * width
+    lens = torch.tensor([min(top, n) for n in (top, 48, 33, 1, 32, 49, 0, 64, 97, 31, 2)[:batch]],
+                        dtype=torch.int32)
+    bt = torch.randperm(batch * width, generator=g).to(torch.int32).view(batch, width)
+    kv = torch.randn(2, batch * width, B, Hk, D, generator=g)
+    kv = kv.to(torch.float8_e4m3fn) if kind == "fp8" else kv.to(dt)
+    q = (3 * torch.randn(batch, Hq, D, generator=g)).to(dt)
+    out = nkv.paged_decode(q.to(dev), kv[0].to(dev), kv[1].to(dev), lens.to(dev), bt.to(dev),
+                           D ** -0.5)
+    torch.cuda.synchronize()
+    ref = paged_decode_ref(q.float(), kv[0].float(), kv[1].float(), lens, bt, D ** -0.5)
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-2  # as above
+
+
 @pytest.mark.parametrize("Hk,D,tokens", [(8, 128, 1), (8, 128, 16383), (8, 128, 16385),
                                          (1, 64, 7), (3, 128, 43691)])
 def test_store_around_its_chunks_per_thread(nkv, dev, Hk, D, tokens):
