@@ -44,6 +44,7 @@
 //    second kernel merges the cut tiles; decode rows (one new token) are streamed by waves of
 //    workgroups of their own, as the decode kernel does.
 #include "decode_stream.h"
+#include "split_share.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -118,18 +119,13 @@ constexpr int kSnap = 2;  // a range never cuts a unit within this many steps of
 // Floats of a partial row: O, m, l, 2 pad.
 constexpr int prefill_part_row(int D) { return D + 4; }
 
-// Cost of one key step of a tile with `rows` rows: its loads and the step's latency, and a share
-// for each wave that has rows to compute. With a smaller base (1 of 5) a range of a sequence's
-// last, partial tile took up to twice the others' time: 1522 tokens in two chunks on 9000 (Hq 16,
-// Hk 8) 207 us, with 5 of 9 155; three chunks and 10 decode rows 70.5, 65.1.
-constexpr int kStepBase = 5;
-constexpr int kFullStep = kStepBase + 4;
 constexpr int kMinRange = 4 * kFullStep;
 // Shortest range over all heads' T tile steps: sqrt(T) / 6 steps. A range's part costs about 7
 // steps to write and merge (100 KB each way), so halving the ranges of a small call gains until
 // its steps take as long: four chunks of 75 - 195 tokens on 2650 (Hq 16, Hk 2) 52.5 -> 46.4 us;
 // no range of a call that fills the chip is touched.
 constexpr float kRangeRoot = 1.f / 6.f;
+// Cost of one key step of a tile with `rows` rows.
 template <int D, bool F8>
 __device__ __forceinline__ int step_cost(int rows) {
   constexpr int kWaveRows = 16 * prefill_row_groups(D, F8);
@@ -146,12 +142,6 @@ __device__ __forceinline__ int tile_steps(int Lq, int Lk, int qt, int t) {
 // stream them as the decode kernel does, bound by the K/V bytes, beside the workgroups that
 // the prompts' tiles keep at the matrix cores. A 192-row tile for one row ran at 5.2 TB/s of
 // K/V (a 256-byte piece of each row and 64 keys in flight a workgroup; decode_stream: 6.5).
-// Cost of a 16-key chunk of one head, in twentieths of a full tile's step: fewer workgroups than
-// their share of the time alone would give them (5 and 3), since the memory serves the rows
-// at its full rate from half the chip's waves while the others compute. 48 rows with two
-// 512-token chunks, at 1, 2, 3, 4, 6: 116, 117, 126, 129, 160 us; 80 rows of 4k - 8k with one:
-// 333, 319, 316, 361; 60 fp8 rows with two: 88, 111, 119, 125.
-constexpr int row_cost(bool F8) { return F8 ? 1 : 2; }
 
 // The ranges of the split launch. The units of a KV head (sequence, tile) stand in one
 // stream, a unit as long as its cost; range w is [w*C, (w+1)*C), with a cut that falls near
@@ -197,15 +187,11 @@ __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
   c.T = T;
   int n_ranges = (int)gridDim.x / Hk;  // of each KV head
   c.row_groups = 0;
-  if constexpr (ROWS) {  // shared out by cost, at least a range of each kind that there is
-    const int rows =
-        __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63) * row_cost(F8) * kFullStep / 20;
-    if (rows > 0) {
-      const int r = (int)((float)n_ranges * (float)rows / (float)(rows + T) + 0.5f);
-      const int r_rows = T > 0 ? min(max(r, 1), n_ranges - 1) : n_ranges;
-      n_ranges -= r_rows;
-      c.row_groups = r_rows * Hk;
-    }
+  if constexpr (ROWS) {
+    const SplitShare share = split_share(
+        n_ranges, __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63), T, F8);
+    n_ranges = share.tiles;
+    c.row_groups = share.rows * Hk;
     if ((int)blockIdx.x < c.row_groups) return false;
   }
   c.group = (int)blockIdx.x - c.row_groups;

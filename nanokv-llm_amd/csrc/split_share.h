@@ -1,0 +1,40 @@
+// How a split launch (prefill.hip) shares its workgroups between the prompts' tiles and the decode
+// rows among them. Plain constexpr C++ that the host plan and the kernels compile, and a test on
+// the CPU.
+#pragma once
+
+#include <stdint.h>
+
+namespace nkv {
+
+// Cost of one key step of a tile: its loads and the step's latency, and a share for each of
+// its four waves that has rows to compute. With a smaller base (1 of 5) a range of a sequence's
+// last, partial tile took up to twice the others' time: 1522 tokens in two chunks on 9000 (Hq 16,
+// Hk 8) 207 us, with 5 of 9 155; three chunks and 10 decode rows 70.5, 65.1.
+constexpr int kStepBase = 5;
+constexpr int kFullStep = kStepBase + 4;
+
+// Cost of a 16-key chunk of a decode row, in twentieths of a full tile's step: fewer workgroups
+// than the rows' share of the time alone would give them (5 and 3), since the memory serves them
+// at its full rate from half the chip's waves while the others compute. 48 rows with two
+// 512-token chunks, at 1, 2, 3, 4, 6: 116, 117, 126, 129, 160 us; 80 rows of 4k - 8k with one:
+// 333, 319, 316, 361; 60 fp8 rows with two: 88, 111, 119, 125.
+constexpr int row_cost(bool f8) { return f8 ? 1 : 2; }
+
+// Workgroups of each KV head for the decode rows and for the tiles.
+struct SplitShare {
+  int rows, tiles;
+};
+// n_ranges workgroups of a KV head shared out by cost over `chunks` chunks of decode rows and
+// tiles of `tile_cost`: at least one for each kind of work that there is, however little of it,
+// since the rows are no tiles and only their own workgroups compute them.
+constexpr SplitShare split_share(int n_ranges, int chunks, int tile_cost, bool f8) {
+  if (chunks <= 0) return SplitShare{0, n_ranges};
+  if (tile_cost <= 0) return SplitShare{n_ranges, 0};
+  const float cost = (float)chunks * ((float)(row_cost(f8) * kFullStep) / 20.f);
+  const int r = (int)((float)n_ranges * cost / (cost + (float)tile_cost) + 0.5f);
+  const int rows = r < 1 ? 1 : r < n_ranges - 1 ? r : n_ranges - 1;
+  return SplitShare{rows, n_ranges - rows};
+}
+
+}  // namespace nkv

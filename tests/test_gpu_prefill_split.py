@@ -111,6 +111,43 @@ def test_split_matches_the_oracle(dev, mix, Hq, Hk, D, kind, B, paged):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "fp8"])
+@pytest.mark.parametrize("rows", [[1], [16], [17], [32], [33], [1, 2], [16, 16], [0, 1, 0]])
+@pytest.mark.parametrize("chunk", [None, (130, 2311)])
+def test_split_computes_the_fewest_short_decode_rows(dev, kind, rows, chunk):
+    """Decode rows of a chunk or two of keys, beside a chunk on a long prefix and alone: a
+    vanishing share of the work, which still has its workgroups."""
+    print(kind, rows, chunk, flush=True)
+    mix = [(1, n) for n in rows] + ([chunk] if chunk else [])
+    q, k, v, cu_q, cu_k, bt = _inputs(dev, mix, 32, 8, 128, kind, 256, True, seed=12)
+    out = _split(dev, q, k, v, cu_q, cu_k, bt, kind, 128 ** -0.5)
+    s = 1 / 16 if kind == "fp8" else 1.0
+    ref = varlen_prefill_ref(q.float(), k.float() * s, v.float() * s, cu_q, cu_k, 128 ** -0.5,
+                             block_tables=bt)
+    assert (out.float().cpu() - ref).abs().max().item() <= TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+def test_attention_beside_a_long_chunk_keeps_a_new_sequences_row(nkv, dev, kind):
+    """A step of a chunk late in a long prompt and the first decode step of a short one, through
+    Attention.forward, whose plan takes the split launch for it."""
+    mix = [(130, 4000), (1, 9)]
+    q, k, v, cu_q, cu_k, bt = _inputs(dev, mix, 32, 8, 128, kind, 256, True, seed=13)
+    t = L.NKV_KV_FP8 if kind == "fp8" else L.NKV_KV_BF16
+    assert L.lib().nkv_prefill_split_plan(2, 131, 130, 4000, 32, 8, 128, t) > 0
+    layer = nkv.Attention(32, 128, 128 ** -0.5, 8, SimpleNamespace(kv_compress_enabled=False), 1)
+    layer.k_cache, layer.v_cache = k.to(dev), v.to(dev)
+    s = layer.k_scale = layer.v_scale = 1 / 16 if kind == "fp8" else 1.0
+    nkv.set_context(False, cu_q.to(dev), cu_k.to(dev), 130, 4000, None, None, bt.to(dev))
+    out = layer(q.to(dev), None, None, 0, kv_stored=True)
+    nkv.reset_context()
+    ref = varlen_prefill_ref(q.float(), k.float() * s, v.float() * s, cu_q, cu_k, 128 ** -0.5,
+                             block_tables=bt)
+    assert (out.float().cpu() - ref).abs().max().item() <= TOL
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["bf16", "fp8"])
 def test_split_takes_invalid_blocks_as_zero_keys(nkv, dev, kind):
     """Table entries outside the pool, and keys past the table's width, are zero keys that take
