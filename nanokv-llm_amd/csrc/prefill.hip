@@ -155,11 +155,12 @@ struct SplitCursor {
 };
 
 // false: nothing to do, or (row_groups > blockIdx.x) the decode rows.
-template <int D, bool F8, bool ROWS>
+template <int D, bool F8, int HP>
 __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
                                             const int32_t* __restrict__ cu_q,
                                             const int32_t* __restrict__ cu_k, int qt, int G,
                                             int Hk, SplitCursor& c) {
+  constexpr bool ROWS = HP > 0;
   const int lane = threadIdx.x & 63;
   int Lq = 0, Lk = 0, cost = 0, incl = 0;
   int chunks = 0;  // lane: of the decode rows
@@ -189,7 +190,7 @@ __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
   c.row_groups = 0;
   if constexpr (ROWS) {
     const SplitShare share = split_share(
-        n_ranges, __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63), T, F8);
+        n_ranges, __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63), T, F8, sa.ncg, HP);
     n_ranges = share.tiles;
     c.row_groups = share.rows * Hk;
     if ((int)blockIdx.x < c.row_groups) return false;
@@ -290,7 +291,7 @@ __device__ __forceinline__ void prefill_body(
   if constexpr (SPLIT) {
     // no unit of this range is cut at its end, unless one below says so
     if (tid == 0) sa.desc[blockIdx.x] = i32x4_t{0, 0, 0, 0};
-    if (!split_begin<D, F8, (HP > 0)>(sa, cu_seqlens_q, cu_seqlens_k, QT, G, Hk, cur)) {
+    if (!split_begin<D, F8, HP>(sa, cu_seqlens_q, cu_seqlens_k, QT, G, Hk, cur)) {
       if constexpr (HP > 0) {
         if ((int)blockIdx.x < cur.row_groups)
           decode_stream<F8, HP, D, H16>(
@@ -1147,13 +1148,15 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
     sa.min_chunks = block_tables ? decode_min_chunks(decode_max_chunks(max_blocks, block_size),
                                                      kMinChunks)
                                  : 0;
-    // a range for each kind of work, dense cache rows, and positions of the decode rows' chunks
-    // in 32 bits
-    if (block_tables && prefill_ranges(n_kv_heads, head_dim) >= 2 &&
-        k_row_stride == (int64_t)n_kv_heads * head_dim &&
+    // dense cache rows, positions of the decode rows' chunks in 32 bits, and workgroups for each
+    // kind of work (otherwise decode rows are tiles)
+    if (block_tables && k_row_stride == (int64_t)n_kv_heads * head_dim &&
         (int64_t)max_blocks * block_size < (1ll << 30) &&
-        (int64_t)block_size * k_row_stride * kEl < (1ll << 31))
+        (int64_t)block_size * k_row_stride * kEl < (1ll << 31)) {
       row_heads = prefill_row_heads<F8>(n_kv_heads, g, head_dim);
+      if (prefill_ranges(n_kv_heads, head_dim) <= row_ranges_least(sa.ncg, row_heads))
+        row_heads = 0;
+    }
     merge_grid = grid * ((tile_rows + kMergeRows - 1) / kMergeRows) +
                  (row_heads ? ((int64_t)n_seqs * n_q_heads + kMergeWaves - 1) / kMergeWaves : 0);
     NKV_REQUIRE(merge_grid < (1ll << 31), NKV_EUNSUPPORTED, "%s: grid too large", what);

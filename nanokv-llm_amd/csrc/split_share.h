@@ -21,19 +21,27 @@ constexpr int kFullStep = kStepBase + 4;
 // 333, 319, 316, 361; 60 fp8 rows with two: 88, 111, 119, 125.
 constexpr int row_cost(bool f8) { return f8 ? 1 : 2; }
 
+// The fewest workgroups of a KV head that the decode rows can have: each brings four waves, and
+// every group of `hp` KV heads and every one of its `ncg` column groups of query heads needs a
+// wave of its own (decode_stream.h).
+constexpr int row_ranges_least(int ncg, int hp) { return (ncg + 4 * hp - 1) / (4 * hp); }
+
 // Workgroups of each KV head for the decode rows and for the tiles.
 struct SplitShare {
   int rows, tiles;
 };
-// n_ranges workgroups of a KV head shared out by cost over `chunks` chunks of decode rows and
-// tiles of `tile_cost`: at least one for each kind of work that there is, however little of it,
-// since the rows are no tiles and only their own workgroups compute them.
-constexpr SplitShare split_share(int n_ranges, int chunks, int tile_cost, bool f8) {
+// n_ranges (more than row_ranges_least) workgroups of a KV head shared out by cost over `chunks`
+// chunks of decode rows and tiles of `tile_cost`: each kind of work that there is has at least
+// the fewest that do it, however little of it there is, since the rows are no tiles and only
+// their own workgroups compute them.
+constexpr SplitShare split_share(int n_ranges, int chunks, int tile_cost, bool f8, int ncg,
+                                 int hp) {
   if (chunks <= 0) return SplitShare{0, n_ranges};
   if (tile_cost <= 0) return SplitShare{n_ranges, 0};
   const float cost = (float)chunks * ((float)(row_cost(f8) * kFullStep) / 20.f);
   const int r = (int)((float)n_ranges * cost / (cost + (float)tile_cost) + 0.5f);
-  const int rows = r < 1 ? 1 : r < n_ranges - 1 ? r : n_ranges - 1;
+  const int least = row_ranges_least(ncg, hp);
+  const int rows = r < least ? least : r < n_ranges - 1 ? r : n_ranges - 1;
   return SplitShare{rows, n_ranges - rows};
 }
 

@@ -128,6 +128,27 @@ def test_split_computes_the_fewest_short_decode_rows(dev, kind, rows, chunk):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,Hq,Hk,D", [
+    ("bf16", 65, 1, 128), ("bf16", 72, 1, 64), ("fp16", 128, 1, 128), ("fp8", 128, 1, 128),
+    ("bf16", 256, 2, 128),
+    # 256 (and 512) KV heads: two workgroups (one) each, fewer than a group of 80 needs
+    ("bf16", 80 * 256, 256, 64), ("fp8", 2 * 512, 512, 64)])
+@pytest.mark.parametrize("mix", [[(1, 200), (40, 1200)], [(40, 1200), (1, 1), (1, 17)],
+                                 [(1, 40), (1, 700)]])
+def test_split_gives_every_column_group_of_the_rows_a_wave(dev, kind, Hq, Hk, D, mix):
+    """Groups of more than 64 query heads take more waves a row than a workgroup has."""
+    if Hk > 2:
+        mix = [(min(a, 3), min(b, 80)) for a, b in mix]
+    print(kind, Hq, Hk, D, mix, flush=True)
+    q, k, v, cu_q, cu_k, bt = _inputs(dev, mix, Hq, Hk, D, kind, 64, True, seed=14)
+    out = _split(dev, q, k, v, cu_q, cu_k, bt, kind, D ** -0.5)
+    s = 1 / 16 if kind == "fp8" else 1.0
+    ref = varlen_prefill_ref(q.float(), k.float() * s, v.float() * s, cu_q, cu_k, D ** -0.5,
+                             block_tables=bt)
+    assert (out.float().cpu() - ref).abs().max().item() <= TOL
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["bf16", "fp8"])
 def test_attention_beside_a_long_chunk_keeps_a_new_sequences_row(nkv, dev, kind):
     """A step of a chunk late in a long prompt and the first decode step of a short one, through
