@@ -334,7 +334,9 @@ int nkv_prefill_varlen_f16(const void* q, int64_t q_row_stride,
  * workgroup takes an equal share of all (sequence, tile, key step) work, whatever the mix of
  * lengths, sequences that bring one token (paged) are streamed as nkv_paged_decode does, and a
  * second kernel merges the tiles and rows whose keys were shared out; the plain entry
- * points give each tile's keys to one workgroup. The workspace (16-byte aligned,
+ * points give each tile's keys to one workgroup, and so does this one where the lengths that
+ * the table's width (n_rows without one) allows could take positions past 32 bits (7e9 tiles x
+ * keys, 16e9 sequences x keys). The workspace (16-byte aligned,
  * nkv_prefill_split_workspace_bytes; independent of the lengths) holds the parts; calls that
  * overlap need one each. */
 size_t nkv_prefill_split_workspace_bytes(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads,

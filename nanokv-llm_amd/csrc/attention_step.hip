@@ -51,16 +51,9 @@ extern "C" int nkv_attention(const nkv_attention_args* a) {
         a->out_row_stride, a->workspace, ws_bytes, a->stream);
   }
   const int32_t max_q = (int32_t)a->max_seqlen_q;
-  if (ws_bytes > 0)
-    return nkv_prefill_varlen_split(
-        (int32_t)a->kv_type, a->q, a->q_row_stride, a->k_cache, a->v_cache, row, row,
-        a->cu_or_lens, a->cu_seqlens_k, a->block_tables, a->bt_row_stride, width, n_seqs, max_q,
-        hq, hk, d, block, n_rows, (float)a->scale, fp8 ? (float)a->k_scale : 1.f,
-        fp8 ? (float)a->v_scale : 1.f, a->out, a->out_row_stride, a->workspace, ws_bytes,
-        a->stream);
-  return prefill_plain((int32_t)a->kv_type, a->q, a->q_row_stride, a->k_cache, a->v_cache, row,
+  return prefill_paged((int32_t)a->kv_type, a->q, a->q_row_stride, a->k_cache, a->v_cache, row,
                        a->cu_or_lens, a->cu_seqlens_k, a->block_tables, a->bt_row_stride, width,
                        n_seqs, a->n_tokens, max_q, hq, hk, d, block, n_rows, (float)a->scale,
                        fp8 ? (float)a->k_scale : 1.f, fp8 ? (float)a->v_scale : 1.f, a->out,
-                       a->out_row_stride, a->stream);
+                       a->out_row_stride, a->workspace, ws_bytes, a->stream);
 }

@@ -26,15 +26,17 @@ void clear_error();
 // Checks the launch just issued on the current thread.
 int check_launch(const char* what);
 
-// The plain paged launches of nkv_prefill_varlen, _f16 and _fp8 by kv_type (rows of row_stride
-// elements), knowing the rows of q: their tiles' size is chosen by it.
-int prefill_plain(int32_t kv_type, const void* q, int64_t q_row_stride, const void* k_cache,
+// The paged launches of nkv_prefill_varlen, _f16 and _fp8 by kv_type (rows of row_stride
+// elements) and, given a workspace, of nkv_prefill_varlen_split, knowing the rows of q: the plain
+// launch's tile size and the split one's bounds go by it.
+int prefill_paged(int32_t kv_type, const void* q, int64_t q_row_stride, const void* k_cache,
                   const void* v_cache, int64_t row_stride, const int32_t* cu_seqlens_q,
                   const int32_t* cu_seqlens_k, const int32_t* block_tables,
                   int64_t bt_row_stride, int32_t max_blocks_per_seq, int32_t n_seqs,
                   int64_t total_q, int32_t max_seqlen_q, int32_t n_q_heads, int32_t n_kv_heads,
                   int32_t head_dim, int32_t block_size, int64_t n_rows, float scale,
-                  float k_scale, float v_scale, void* out, int64_t out_row_stride, void* stream);
+                  float k_scale, float v_scale, void* out, int64_t out_row_stride,
+                  void* workspace, size_t workspace_bytes, void* stream);
 
 // Compute units of the current device (cached per device; 256 when it cannot be queried).
 int device_cus();

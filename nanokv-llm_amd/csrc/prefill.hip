@@ -982,6 +982,13 @@ static int prefill_row_heads(int32_t n_kv_heads, int32_t G, int32_t head_dim) {
   return 1;
 }
 
+// Tiles of qt queries that a batch can have at most (total_q < 0: its rows are not known).
+static int64_t split_most_tiles(int64_t n_seqs, int64_t total_q, int64_t max_seqlen_q,
+                                int64_t qt) {
+  const int64_t most = n_seqs * ((max_seqlen_q + qt - 1) / qt);
+  return total_q < 0 ? most : std::min(most, total_q / qt + n_seqs);
+}
+
 // What the host knows of a batch's composition: as few prompts as could bring its rows of q
 // (total_q; every sequence's max_seqlen_q where it is not known), the others being decode rows.
 struct BatchMix {
@@ -1049,13 +1056,13 @@ static bool prefill_split_wins(int32_t n_seqs, int64_t total_q, int32_t max_seql
   const int64_t tiles_max = (max_seqlen_q + qt - 1) / qt;
   // every range counts the tiles of the sequences before it: not for long prompts (whose
   // tiles fill the chip anyway)
-  if (tiles_max > 96 || max_seqlen_k < max_seqlen_q) return false;
+  if (tiles_max > 96 || max_seqlen_k < max_seqlen_q ||
+      !split_fits(n_seqs, split_most_tiles(n_seqs, total_q, max_seqlen_q, qt), max_seqlen_k))
+    return false;
   const BatchMix m = batch_mix(n_seqs, total_q, max_seqlen_q);
   const int64_t tiles = std::min(m.prompts * tiles_max, m.prompt_rows / qt + m.prompts);
   const int64_t rows = m.rows;
   const double steps = (max_seqlen_k + kStep - 1) / kStep;
-  // positions of the stream are 32 bits
-  if ((tiles + rows) * steps * 8 >= 2147483648.0) return false;
   const double per_range = 1.0 / prefill_ranges(n_kv_heads, head_dim);
   const double seen = 1.0 - 0.5 * max_seqlen_q / max_seqlen_k;  // causal: of a prompt's own keys
   const double tile_steps = tiles * steps * seen * per_range * (n_seqs == 1 ? 1.0 : 0.5);
@@ -1065,7 +1072,8 @@ static bool prefill_split_wins(int32_t n_seqs, int64_t total_q, int32_t max_seql
          35.0 + dim * (1.5 * tile_steps + 0.25 * row_steps);
 }
 
-// `split`: a split launch over `workspace`; a plain one otherwise.
+// `split`: a split launch over `workspace` where the lengths that a table row (or the K/V rows)
+// can have leave its positions in 32 bits; a plain one otherwise.
 template <bool F8, bool H16 = false>
 static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cache,
                           const void* v_cache, int64_t k_row_stride, int64_t v_row_stride,
@@ -1119,6 +1127,11 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
   // paged: valid block ids are [0, n_rows / block_size); contiguous: valid rows
   const int32_t n_limit = (int32_t)std::min<int64_t>(block_tables ? n_rows / block_size : n_rows,
                                                      INT32_MAX);
+  if (split)
+    split = split_fits(n_seqs,
+                       split_most_tiles(n_seqs, total_q, max_seqlen_q,
+                                        prefill_tile_rows(head_dim, F8) / g),
+                       block_tables ? (int64_t)max_blocks * block_size : n_rows);
   const int groups = split ? prefill_row_groups(head_dim, F8)
                            : prefill_groups(n_seqs, total_q, max_seqlen_q, n_kv_heads, g,
                                             head_dim, F8);
@@ -1218,20 +1231,21 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
 }  // namespace nkv
 
 namespace nkv {
-int prefill_plain(int32_t kv_type, const void* q, int64_t q_row_stride, const void* k_cache,
+int prefill_paged(int32_t kv_type, const void* q, int64_t q_row_stride, const void* k_cache,
                   const void* v_cache, int64_t row_stride, const int32_t* cu_seqlens_q,
                   const int32_t* cu_seqlens_k, const int32_t* block_tables,
                   int64_t bt_row_stride, int32_t max_blocks_per_seq, int32_t n_seqs,
                   int64_t total_q, int32_t max_seqlen_q, int32_t n_q_heads, int32_t n_kv_heads,
                   int32_t head_dim, int32_t block_size, int64_t n_rows, float scale,
                   float k_scale, float v_scale, void* out, int64_t out_row_stride,
-                  void* stream) {
+                  void* workspace, size_t workspace_bytes, void* stream) {
 #define NKV_PREFILL_ANY(...)                                                                   \
   prefill_launch<__VA_ARGS__>(q, q_row_stride, k_cache, v_cache, row_stride, row_stride,       \
                               cu_seqlens_q, cu_seqlens_k, block_tables, bt_row_stride,         \
                               max_blocks_per_seq, n_seqs, max_seqlen_q, n_q_heads, n_kv_heads, \
                               head_dim, block_size, n_rows, scale, k_scale, v_scale, out,      \
-                              out_row_stride, stream, total_q)
+                              out_row_stride, stream, total_q, workspace_bytes > 0, workspace, \
+                              workspace_bytes)
   if (kv_type == NKV_KV_FP8) return NKV_PREFILL_ANY(true);
   if (kv_type == NKV_KV_F16) return NKV_PREFILL_ANY(false, true);
   return NKV_PREFILL_ANY(false);

@@ -45,4 +45,15 @@ constexpr SplitShare split_share(int n_ranges, int chunks, int tile_cost, bool f
   return SplitShare{rows, n_ranges - rows};
 }
 
+// Whether a split launch's positions fit 32 bits with n_seqs sequences of up to `keys` keys (whose
+// lengths are 32 bits) and `tiles` tiles of theirs: the tiles' key steps by cost, of which a range's
+// end can lie as far past the last as a range is long, and the decode rows' chunks.
+constexpr bool split_fits(int64_t n_seqs, int64_t tiles, int64_t keys) {
+  constexpr int64_t most = 1000000000;
+  if (n_seqs > most || tiles > most) return false;  // the products below stay within 64 bits
+  if (keys > INT32_MAX) keys = INT32_MAX;
+  const int64_t steps = keys > 64 ? (keys + 63) / 64 : 1;
+  return tiles * steps * kFullStep <= most && n_seqs * ((keys + 15) / 16) <= most;
+}
+
 }  // namespace nkv

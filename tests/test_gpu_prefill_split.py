@@ -51,7 +51,7 @@ def _inputs(dev, mix, Hq, Hk, D, kind, B, paged, seed):
     return q, kv[0], kv[1], cs(lq), cs(lk), bt
 
 
-def _split(dev, q, k, v, cu_q, cu_k, bt, kind, scale):
+def _split(dev, q, k, v, cu_q, cu_k, bt, kind, scale, used=None):
     N, Hq, D = q.shape
     t = {"bf16": L.NKV_KV_BF16, "fp16": L.NKV_KV_F16, "fp8": L.NKV_KV_FP8}[kind]
     Hk = k.size(-2)
@@ -74,6 +74,8 @@ def _split(dev, q, k, v, cu_q, cu_k, bt, kind, scale):
         s, s, out.data_ptr(), out.stride(0), ws.data_ptr(), ws.numel(), L.stream_of(d[0])),
         "prefill_varlen_split")
     torch.cuda.synchronize()
+    if used is not None:
+        used.append(bool((ws != 0xff).any()))
     return out
 
 
@@ -186,6 +188,23 @@ def test_split_takes_invalid_blocks_as_zero_keys(nkv, dev, kind):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("width,split", [(16, True), (5 << 20, False)])
+def test_split_leaves_tables_beyond_32_bit_positions_to_the_plain_launch(nkv, dev, width, split):
+    """A table whose rows could hold more keys than positions (1.3e9 of 256 blocks): the plain
+    launch's own bits, and the workspace not touched."""
+    q, k, v, cu_q, cu_k, bt = _inputs(dev, [(200, 900), (1, 40)], 8, 4, 128, "bf16", 256, True,
+                                      seed=15)
+    wide = torch.full((2, width), -1, dtype=torch.int32)
+    wide[:, :bt.size(1)] = bt
+    used = []
+    out = _split(dev, q, k, v, cu_q, cu_k, wide, "bf16", 128 ** -0.5, used)
+    plain = nkv.varlen_prefill(*(x.to(dev) for x in (q, k, v, cu_q, cu_k)), 200, 128 ** -0.5,
+                               block_tables=bt.to(dev))
+    assert used == [split] and torch.equal(out, plain) == (not split)
+    assert (out.float() - plain.float()).abs().max().item() <= 2 ** -7  # |out| < 2: half an ulp
+
+
+@pytest.mark.gpu
 def test_attention_takes_a_long_prefix_to_the_split_launch(nkv, dev):
     """Attention.forward against the plain launch: two orders of the same sums, each weight
     and output rounded to bf16 (2^-8 relative, |out| < 1 here); then captured in a graph and
@@ -255,6 +274,9 @@ def test_split_plan_and_arguments_on_the_host():
     assert plan(1, 512, 512, 0, 32, 8, 128, L.NKV_KV_BF16) == 0
     assert plan(0, 0, 0, 0, 32, 8, 128, L.NKV_KV_BF16) == 0
     assert plan(1, 512, 512, 12800, 30, 8, 128, L.NKV_KV_BF16) == 0
+    # positions in 32 bits: 200 rows of a million keys, not 2000 of eight
+    assert plan(200, 711, 512, 1 << 20, 32, 8, 128, L.NKV_KV_BF16) == size(200)
+    assert plan(2000, 2511, 512, 1 << 23, 32, 8, 128, L.NKV_KV_BF16) == 0
 
     def call(kv_type=L.NKV_KV_BF16, ws=1 << 12, nbytes=full, bt=1 << 12):
         return lib.nkv_prefill_varlen_split(

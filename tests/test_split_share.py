@@ -18,6 +18,9 @@ extern "C" int share(int n, int chunks, int tiles, int f8, int ncg, int hp) {
   const nkv::SplitShare s = nkv::split_share(n, chunks, tiles, f8 != 0, ncg, hp);
   return s.rows * 65536 + s.tiles;
 }
+extern "C" int fits(int64_t n_seqs, int64_t tiles, int64_t keys) {
+  return nkv::split_fits(n_seqs, tiles, keys);
+}
 """
 
 
@@ -31,7 +34,9 @@ def lib(tmp_path_factory):
     src.write_text(SOURCE)
     subprocess.run([gxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-fPIC", "-shared", "-I", CSRC,
                     str(src), "-o", str(so)], check=True)
-    return C.CDLL(str(so))
+    lib = C.CDLL(str(so))
+    lib.fits.argtypes = [C.c_int64] * 3
+    return lib
 
 
 def _instances(cus=256):
@@ -51,8 +56,8 @@ def _instances(cus=256):
 @pytest.mark.parametrize("f8", [0, 1])
 def test_every_kind_of_work_gets_workgroups(lib, f8):
     for n, hk, ncg, hp in _instances():
-        for chunks in [*range(0, 41), 1000, 10 ** 6]:
-            for tiles in (0, 5, 9, 90, 7000, 10 ** 6, 10 ** 8):
+        for chunks in [*range(0, 41), 1000, 10 ** 6, 119304648, 10 ** 9]:
+            for tiles in (0, 5, 9, 90, 7000, 10 ** 6, 10 ** 9):
                 if chunks == tiles == 0:
                     continue
                 s = lib.share(n, chunks, tiles, f8, ncg, hp)
@@ -62,3 +67,22 @@ def test_every_kind_of_work_gets_workgroups(lib, f8):
                 assert (rows > 0) == (chunks > 0) and (left > 0) == (tiles > 0), at
                 # waves of each group of KV heads and columns
                 assert chunks == 0 or 4 * rows * hk // (hk * ncg // hp) >= 1, at
+
+
+def test_positions_of_a_stream_that_fits_stay_within_32_bits(lib):
+    """The tiles' cost, a range's end up to a range past it, and the decode rows' chunks."""
+    at_limit, top = 0, 2 ** 31 - 1
+    for n_seqs in (1, 7, 1000, top):
+        for tiles in (1, 96, 10 ** 5, 10 ** 9, 2 ** 40, 2 ** 62):
+            for bits in range(4, 36):
+                for keys in (2 ** bits - 1, 2 ** bits, 2 ** bits + 1):
+                    cost = max(tiles * -(-min(keys, top) // 64) * 9,
+                               n_seqs * -(-min(keys, top) // 16))
+                    if lib.fits(n_seqs, tiles, keys):
+                        assert 2 * cost + 2 ** 20 < 2 ** 31, (n_seqs, tiles, keys)
+                        at_limit += cost > 2 ** 28
+                    else:  # nothing far from the limit is turned away
+                        assert cost > 2 ** 29, (n_seqs, tiles, keys)
+    assert at_limit > 0
+    # 2000 rows of a million keys (shared blocks): within; 200000: beyond
+    assert lib.fits(2000, 2100, 1 << 20) == 1 and lib.fits(200000, 200100, 1 << 20) == 0
