@@ -77,12 +77,15 @@ struct DecodeSeqs {
 };
 // The sequences of a variable-length batch that bring one new token (the others have no chunk
 // here): row cu_q[s] of q and out. Keys past the table or in an invalid block are zeros that
-// take their weight, as everywhere in such a batch.
+// take their weight, as everywhere in such a batch: those in a block are chunks like the others,
+// those past the table's max_tokens are weighed by the combine, so that no row has more
+// partials than its table's width allows.
 struct OneRowSeqs {
   static constexpr bool kZeroInvalid = true;
   const int32_t* __restrict__ cu_q;
   const int32_t* __restrict__ cu_k;
   int32_t batch;
+  int32_t max_tokens;
   __device__ __forceinline__ int keys(int s) const {
     return cu_q[s + 1] - cu_q[s] == 1 ? cu_k[s + 1] - cu_k[s] : 0;
   }
@@ -90,17 +93,15 @@ struct OneRowSeqs {
 };
 
 // Chunks of a sequence of ctx keys.
-template <typename Seqs>
 __device__ __forceinline__ int seq_chunks(int ctx, int max_tokens) {
-  if constexpr (!Seqs::kZeroInvalid) NKV_DBG(ctx < 0 || ctx > max_tokens, NKV_DEBUG_LENGTH);
-  const int n = Seqs::kZeroInvalid ? ctx : min(ctx, max_tokens);
-  return n > 0 ? (n + kChunk - 1) / kChunk : 0;
+  NKV_DBG(ctx < 0 || ctx > max_tokens, NKV_DEBUG_LENGTH);
+  return ctx > 0 ? (min(ctx, max_tokens) + kChunk - 1) / kChunk : 0;
 }
 template <typename Seqs>
 __device__ __forceinline__ void seq_load(SeqCursor& c, const Seqs& seqs, int max_tokens) {
   const int s = c.cb + (int)(threadIdx.x & 63);
   c.ctx = s < seqs.batch ? seqs.keys(s) : 0;
-  c.nc = seq_chunks<Seqs>(c.ctx, max_tokens);
+  c.nc = seq_chunks(c.ctx, max_tokens);
   c.incl = wave_incl_scan(c.nc);
   c.tot = __builtin_amdgcn_readlane(c.incl, 63);
 }
@@ -211,7 +212,7 @@ __device__ __forceinline__ void decode_stream(
     int more = 0;
 #pragma unroll 4
     for (int s = 64 + lane; s < batch; s += 64)
-      more += seq_chunks<Seqs>(seqs.keys(s), max_tokens);
+      more += seq_chunks(seqs.keys(s), max_tokens);
     T += __builtin_amdgcn_readlane(wave_incl_scan(more), 63);
   }
   // equal ranges over the resident waves, at least min_chunks (which keeps every
@@ -283,9 +284,6 @@ __device__ __forceinline__ void decode_stream(
           NKV_DBG(id < 0 || id >= n_blocks, NKV_DEBUG_BLOCK);  // every block here is needed
           blk_id = (id >= 0 && id < n_blocks) ? id : -1;
         }
-        if constexpr (Seqs::kZeroInvalid)
-          NKV_DBG(bi >= max_blocks && bi * block_size < min((wlo + wn) * kChunk, ctx),
-                  NKV_DEBUG_LENGTH);
       }
 
       u32x4_t kreg[kRing][kLoads];
@@ -474,6 +472,7 @@ __device__ __forceinline__ void decode_combine(
     const float* __restrict__ part, const i32x4v_t* __restrict__ desc,
     bf16_t* __restrict__ out, int64_t out_row_stride) {
   static_assert(decode_dim_ok(D), "head_dim 64, 128 or 256");
+  static_assert(WAVES == 1 || !Seqs::kZeroInvalid, "each wave would weigh the keys past the table");
   constexpr int N = D / 64;
   constexpr int kPartRow = part_row(D);
   constexpr int kPer = (kMaxSlots + 64 * WAVES - 1) / (64 * WAVES);  // (m, l) pairs a lane holds
@@ -527,6 +526,11 @@ __device__ __forceinline__ void decode_combine(
 #pragma unroll
   for (int k = 1; k < kPer; ++k) M = fmaxf(M, ml[k].x);
   M = wave_max(M);
+  int past = 0;  // zero keys past the table: score 0
+  if constexpr (Seqs::kZeroInvalid) {
+    past = max(ctx - seqs.max_tokens, 0);
+    if (past > 0) M = fmaxf(M, 0.f);
+  }
   float w[kPer], L = 0.f;
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
@@ -534,6 +538,7 @@ __device__ __forceinline__ void decode_combine(
     L += w[k] * ml[k].y;
   }
   L = wave_sum(L);
+  if (past > 0) L = fmaf((float)past, fast_exp2(-M), L);
 #pragma unroll
   for (int u = 0; u < kFirst; ++u) {
     const float wu = __shfl(w[0], u, 64);

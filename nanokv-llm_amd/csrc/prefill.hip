@@ -113,6 +113,7 @@ struct SplitArgs {
   int32_t min_chunks;  // descriptors and partial rows (decode_stream.h)
   i32x4v_t* row_desc;
   float* row_part;
+  int32_t max_tokens;  // keys that a table row holds
 };
 constexpr int kSnap = 2;  // a range never cuts a unit within this many steps of its ends
 
@@ -174,7 +175,7 @@ __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
       NKV_DBG(blockIdx.x == 0 && (Lq < 0 || Lk < 0 || Lq > Lk), NKV_DEBUG_LENGTH);
     }
     if (ROWS && Lq == 1) {
-      chunks += (max(Lk, 0) + kChunk - 1) / kChunk;
+      chunks += seq_chunks(Lk, sa.max_tokens);
       Lq = 0;
     }
     cost = 0;
@@ -295,11 +296,11 @@ __device__ __forceinline__ void prefill_body(
       if constexpr (HP > 0) {
         if ((int)blockIdx.x < cur.row_groups)
           decode_stream<F8, HP, D, H16>(
-              OneRowSeqs{cu_seqlens_q, cu_seqlens_k, sa.n_seqs}, (int)blockIdx.x * 4 + wave,
-              cur.row_groups * 4, reinterpret_cast<bf16_t*>(ring + wave * kRowLds), q,
-              q_row_stride, k_cache, v_cache, block_tables, bt_row_stride, Hk, G, sa.ncg,
-              block_size, max_blocks, n_limit, sa.min_chunks, scale_log2, v_scale, sa.row_part,
-              sa.row_desc);
+              OneRowSeqs{cu_seqlens_q, cu_seqlens_k, sa.n_seqs, sa.max_tokens},
+              (int)blockIdx.x * 4 + wave, cur.row_groups * 4,
+              reinterpret_cast<bf16_t*>(ring + wave * kRowLds), q, q_row_stride, k_cache, v_cache,
+              block_tables, bt_row_stride, Hk, G, sa.ncg, block_size, max_blocks, n_limit,
+              sa.min_chunks, scale_log2, v_scale, sa.row_part, sa.row_desc);
       }
       return;  // uniform
     }
@@ -852,8 +853,9 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(
     const int id = ((int)blockIdx.x - n_tile_blocks) * kMergeWaves + wave;
     const int b = id / Hq;
     if (b < sa.n_seqs && cu_q[b + 1] - cu_q[b] == 1)  // uniform over the wave
-      decode_combine<D, H16, 1>(OneRowSeqs{cu_q, cu_k, sa.n_seqs}, b, id - b * Hq, Hq, Hk,
-                                sa.ncg, sa.row_part, sa.row_desc, out, out_row_stride);
+      decode_combine<D, H16, 1>(OneRowSeqs{cu_q, cu_k, sa.n_seqs, sa.max_tokens}, b,
+                                id - b * Hq, Hq, Hk, sa.ncg, sa.row_part, sa.row_desc, out,
+                                out_row_stride);
     return;
   }
   const int x = blockIdx.x % n_groups;
@@ -1166,6 +1168,7 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
     if (block_tables && k_row_stride == (int64_t)n_kv_heads * head_dim &&
         (int64_t)max_blocks * block_size < (1ll << 30) &&
         (int64_t)block_size * k_row_stride * kEl < (1ll << 31)) {
+      sa.max_tokens = max_blocks * block_size;
       row_heads = prefill_row_heads<F8>(n_kv_heads, g, head_dim);
       if (prefill_ranges(n_kv_heads, head_dim) <= row_ranges_least(sa.ncg, row_heads))
         row_heads = 0;

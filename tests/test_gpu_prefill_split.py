@@ -188,6 +188,29 @@ def test_split_takes_invalid_blocks_as_zero_keys(nkv, dev, kind):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "fp8"])
+@pytest.mark.parametrize("prompt", [None, (60, 500)])
+def test_split_weighs_every_key_past_a_narrow_table(nkv, dev, kind, prompt):
+    """Decode rows of up to 30000 keys over a table of 160: the keys past it are zeros that take
+    their weight, all of them, however many ranges they would have made (the plain launch's
+    results from two orders of the same sums: a bf16 ulp, 2^-6 where 2 <= |out| < 4, as the row
+    of 160 keys with these peaked scores has)."""
+    mix = [(1, 30000), (1, 9000), (1, 161), (1, 160)] + ([prompt] if prompt else [])
+    g = torch.Generator().manual_seed(16)
+    q, k, v, cu_q, cu_k, bt = _inputs(dev, [(a, min(b, 160)) for a, b in mix[:4]] + mix[4:],
+                                      16, 4, 128, kind, 16, True, seed=16)
+    q = (3 * torch.randn(q.shape, generator=g)).to(q.dtype)  # the keys there weigh as much
+    cu_k = torch.tensor([0] + [b for _, b in mix]).cumsum(0).to(torch.int32)
+    bt = bt[:, :10].contiguous()
+    out = _split(dev, q, k, v, cu_q, cu_k, bt, kind, 128 ** -0.5)
+    s = 1 / 16 if kind == "fp8" else 1.0
+    max_q = 60 if prompt else 1
+    plain = nkv.varlen_prefill(*(x.to(dev) for x in (q, k, v, cu_q, cu_k)), max_q, 128 ** -0.5,
+                               block_tables=bt.to(dev), k_scale=s, v_scale=s)
+    assert (out.float() - plain.float()).abs().max().item() <= 2 ** -6
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("width,split", [(16, True), (5 << 20, False)])
 def test_split_leaves_tables_beyond_32_bit_positions_to_the_plain_launch(nkv, dev, width, split):
     """A table whose rows could hold more keys than positions (1.3e9 of 256 blocks): the plain
