@@ -1351,6 +1351,7 @@ extern "C" int nkv_prefill_varlen_split(int32_t kv_type, const void* q, int64_t 
                                         size_t workspace_bytes, void* stream) {
   using namespace nkv;
   clear_error();
+  if (kv_type != NKV_KV_FP8) k_scale = v_scale = 1.f;
 #define NKV_PREFILL_SPLIT(...)                                                                 \
   prefill_launch<__VA_ARGS__>(q, q_row_stride, k_cache, v_cache, k_row_stride, v_row_stride,   \
                               cu_seqlens_q, cu_seqlens_k, block_tables, bt_row_stride,         \

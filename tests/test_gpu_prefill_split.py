@@ -51,13 +51,13 @@ def _inputs(dev, mix, Hq, Hk, D, kind, B, paged, seed):
     return q, kv[0], kv[1], cs(lq), cs(lk), bt
 
 
-def _split(dev, q, k, v, cu_q, cu_k, bt, kind, scale, used=None):
+def _split(dev, q, k, v, cu_q, cu_k, bt, kind, scale, used=None, scales=None):
     N, Hq, D = q.shape
     t = {"bf16": L.NKV_KV_BF16, "fp16": L.NKV_KV_F16, "fp8": L.NKV_KV_FP8}[kind]
     Hk = k.size(-2)
     n_rows = k.size(0) * (k.size(1) if bt is not None else 1)
     ks, vs = (k.stride(0), v.stride(0)) if bt is None else (Hk * D, Hk * D)
-    s = 1 / 16 if kind == "fp8" else 1.0
+    s = scales or (1 / 16 if kind == "fp8" else 1.0)
     d = [x.to(dev) if x is not None else None for x in (q, k, cu_q, cu_k, bt)]
     # a strided V stays strided on the device
     vd = v.to(dev) if v.is_contiguous() else \
@@ -211,6 +211,15 @@ def test_split_weighs_every_key_past_a_narrow_table(nkv, dev, kind, prompt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,scales", [("bf16", 3.0), ("fp16", -1.0)])
+def test_split_uses_the_scales_of_an_fp8_pool_only(dev, kind, scales):
+    """Finished tiles, merged ones and decode rows alike."""
+    q, k, v, cu_q, cu_k, bt = _inputs(dev, MIXES["mixed"], 16, 4, 128, kind, 64, True, seed=17)
+    args = (dev, q, k, v, cu_q, cu_k, bt, kind, 128 ** -0.5)
+    assert torch.equal(_split(*args, scales=scales), _split(*args))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("width,split", [(16, True), (5 << 20, False)])
 def test_split_leaves_tables_beyond_32_bit_positions_to_the_plain_launch(nkv, dev, width, split):
     """A table whose rows could hold more keys than positions (1.3e9 of 256 blocks): the plain
@@ -301,11 +310,14 @@ def test_split_plan_and_arguments_on_the_host():
     assert plan(200, 711, 512, 1 << 20, 32, 8, 128, L.NKV_KV_BF16) == size(200)
     assert plan(2000, 2511, 512, 1 << 23, 32, 8, 128, L.NKV_KV_BF16) == 0
 
-    def call(kv_type=L.NKV_KV_BF16, ws=1 << 12, nbytes=full, bt=1 << 12):
+    def call(kv_type=L.NKV_KV_BF16, ws=1 << 12, nbytes=full, bt=1 << 12, scale=1.0):
         return lib.nkv_prefill_varlen_split(
             kv_type, 1 << 12, 32 * 128, 1 << 12, 1 << 12, 8 * 128, 8 * 128, 1 << 12, 1 << 12, bt,
-            4, 4, 1, 16, 32, 8, 128, 256, 4 * 256, 1.0, 1.0, 1.0, 1 << 12, 32 * 128, ws, nbytes,
+            4, 4, 1, 16, 32, 8, 128, 256, 4 * 256, 1.0, scale, scale, 1 << 12, 32 * 128, ws, nbytes,
             None)
     assert call(kv_type=3) == -1
     assert call(ws=None) == -3 and call(ws=(1 << 12) + 8) == -3 and call(nbytes=full - 1) == -3
     assert call(kv_type=L.NKV_KV_FP8, bt=None) == -1  # fp8 rows are paged
+    # scales belong to fp8 rows: others get to the workspace's check whatever they are
+    assert call(scale=0.0, ws=None) == -3
+    assert call(kv_type=L.NKV_KV_FP8, scale=0.0, ws=None) == -1
