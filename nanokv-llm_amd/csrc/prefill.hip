@@ -13,7 +13,7 @@
 //    heads (GQA sharing). Wave w owns up to three 16-row groups at head_dim 128
 //    (R = 192), two at 64 and in the fp8 instance (R = 128), one at 256
 //    (R = 64, and the 128 KiB ring leaves one workgroup per CU); fewer where
-//    the batch has few tiles (prefill_groups). head_dim D is 64, 128 or 256 (a
+//    the batch has few tiles (plain_groups). head_dim D is 64, 128 or 256 (a
 //    template parameter).
 //  * Keys advance in 64-key steps. Each step's K and V tiles (2 x 16 KiB at
 //    D = 128) go from HBM straight into LDS with gfx950's 16-byte buffer-load-to-LDS
@@ -44,7 +44,7 @@
 //    second kernel merges the cut tiles; decode rows (one new token) are streamed by waves of
 //    workgroups of their own, as the decode kernel does.
 #include "decode_stream.h"
-#include "split_share.h"
+#include "prefill_rules.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -991,52 +991,6 @@ static int64_t split_most_tiles(int64_t n_seqs, int64_t total_q, int64_t max_seq
   return total_q < 0 ? most : std::min(most, total_q / qt + n_seqs);
 }
 
-// What the host knows of a batch's composition: as few prompts as could bring its rows of q
-// (total_q; every sequence's max_seqlen_q where it is not known), the others being decode rows.
-struct BatchMix {
-  int64_t prompts, rows, prompt_rows;  // prompts, decode rows, the prompts' rows of q
-};
-static BatchMix batch_mix(int64_t n_seqs, int64_t total_q, int64_t max_seqlen_q) {
-  if (total_q < 0) total_q = n_seqs * max_seqlen_q;
-  const int64_t more = std::max<int64_t>(0, total_q - n_seqs);  // beyond one token each
-  BatchMix m;
-  m.prompts = max_seqlen_q > 1
-                  ? std::min(n_seqs, (more + max_seqlen_q - 2) / (max_seqlen_q - 1))
-                  : 0;
-  m.rows = n_seqs - m.prompts;
-  m.prompt_rows = total_q - m.rows;
-  return m;
-}
-
-// Row groups per wave of a plain launch (every number gives the same bits). More rows a tile
-// need fewer reads of K and V from LDS per MFMA, fewer leave more workgroups to overlap, and a
-// workgroup's key step takes 1.15 us with one, 1.26 with two, 1.75 with three while the chip is
-// not full. Measured (Hq 32, Hk 8; 1 / 2 / 3 groups, us; workgroups as with three):
-//   a prompt of 333 (56 workgroups)     11.2 /  14.4 /  20.2
-//   of 1500 (256)                       33.4 /  38.0 /  51.6
-//   of 3000 (504)                       95.5 /  80.2 /  98.3
-//   four chunks of 2048 on 6000 (1376)  1053 /   809 /   841
-//   16 prompts up to 1500 (3144)         305 /   229 /   241
-//   16 prompts up to 4096 (8472)        1682 /  1315 /  1294
-//   80 decode rows, a prompt of 300      34.3 /  51.0 /  46.9 (a row's tile is a row)
-static int prefill_groups(int64_t n_seqs, int64_t total_q, int64_t max_seqlen_q,
-                          int32_t n_kv_heads, int g, int32_t head_dim, bool f8) {
-  const int most = prefill_row_groups(head_dim, f8);
-  const BatchMix m = batch_mix(n_seqs, total_q, max_seqlen_q);
-  const int64_t qt = 64 * most / g;
-  const int64_t tiles =
-      std::min(m.prompts * ((max_seqlen_q + qt - 1) / qt), m.prompt_rows / qt + m.prompts);
-  const int64_t groups = (tiles + m.rows) * n_kv_heads;
-  const int64_t cus = device_cus();
-  const int want = g <= 64 && (groups <= cus || m.rows >= tiles) ? 1
-                   : groups <= 16 * cus                          ? std::min(most, 2)
-                                                                 : most;
-  // every sequence's tiles are launched as for the longest: more of them only while the empty
-  // ones are few, and no launch grows past what the largest tiles would take beyond that
-  const int64_t q = 64 * want / g;
-  return n_seqs * ((max_seqlen_q + q - 1) / q) * n_kv_heads <= (1 << 16) ? want : most;
-}
-
 // Whether the split launch is the faster one, from what the host knows of the lengths and the
 // batch's mix. In us, fitted to both sides' times of 200 random steps (1 - 104 sequences, 1 -
 // 3000 new tokens, contexts of up to 16k, every KV type):
@@ -1135,8 +1089,8 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
                                         prefill_tile_rows(head_dim, F8) / g),
                        block_tables ? (int64_t)max_blocks * block_size : n_rows);
   const int groups = split ? prefill_row_groups(head_dim, F8)
-                           : prefill_groups(n_seqs, total_q, max_seqlen_q, n_kv_heads, g,
-                                            head_dim, F8);
+                           : plain_groups(n_seqs, total_q, max_seqlen_q, n_kv_heads, g,
+                                          prefill_row_groups(head_dim, F8), device_cus());
   const int tile_rows = 64 * groups;
   const int qt = tile_rows / g;
   const int n_tiles = (max_seqlen_q + qt - 1) / qt;

@@ -1,0 +1,123 @@
+// The rules by which the variable-length launches (prefill.hip) are chosen and share out their
+// work: a plain launch's tile size, and a split one's workgroups between the prompts' tiles and
+// the decode rows among them. Plain constexpr C++ that the host and the kernels compile, and a
+// test on the CPU.
+#pragma once
+
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace nkv {
+
+// What the host knows of a batch's composition: as few prompts as could bring its rows of q
+// (total_q; every sequence's max_seqlen_q where it is not known), the others being decode rows.
+struct BatchMix {
+  int64_t prompts, rows, prompt_rows;  // prompts, decode rows, the prompts' rows of q
+};
+constexpr BatchMix batch_mix(int64_t n_seqs, int64_t total_q, int64_t max_seqlen_q) {
+  if (total_q < 0) total_q = n_seqs * max_seqlen_q;
+  const int64_t more = std::max<int64_t>(0, total_q - n_seqs);  // beyond one token each
+  BatchMix m{};
+  m.prompts = max_seqlen_q > 1
+                  ? std::min(n_seqs, (more + max_seqlen_q - 2) / (max_seqlen_q - 1))
+                  : 0;
+  m.rows = n_seqs - m.prompts;
+  m.prompt_rows = total_q - m.rows;
+  return m;
+}
+
+// Row groups per wave of a plain launch, up to `most` (every number gives the same bits). More rows
+// a tile need fewer reads of K and V from LDS per MFMA, fewer leave more workgroups to overlap, and
+// a workgroup's key step takes 1.15 us with one, 1.26 with two, 1.75 with three while the chip is
+// not full. Measured (Hq 32, Hk 8; 1 / 2 / 3 groups, us; workgroups as with three):
+//   a prompt of 333 (56 workgroups)     11.2 /  14.4 /  20.2
+//   of 1500 (256)                       33.4 /  38.0 /  51.6
+//   of 3000 (504)                       95.5 /  80.2 /  98.3
+//   four chunks of 2048 on 6000 (1376)  1053 /   809 /   841
+//   16 prompts up to 1500 (3144)         305 /   229 /   241
+//   16 prompts up to 4096 (8472)        1682 /  1315 /  1294
+//   80 decode rows, a prompt of 300      34.3 /  51.0 /  46.9 (a row's tile is a row)
+// Large GQA groups g leave a part of a tile's rows unused, more of a small tile's (a group of 48
+// fills 192 rows, 96 of 128): the lines lie at the tiles that there are of each size, and on a
+// full chip two groups need 7/8 of the use that `most` makes of its rows (1 / 2 / 3, us):
+//   Hq 33, Hk 1 (64, 99, 165 rows used): 600 15.1 / 17.7 / 25.0, 1300 44.9 / 33.2 / 44.3,
+//     16 prompts up to 1500 168 / 97 / 102
+//   Hq 48, Hk 1 (48, 96, 192): 1300 45.4 / 37.1 / 46.4, 2000 88.0 / 73.9 / 68.2, 6 of 1000 152 /
+//     118 / 97
+//   Hq 96, Hk 1 (-, 96, 192): 600 - / 23.8 / 28.0, 1300 - / 64.1 / 52.9, 6 of 1000 - / 235 / 180
+constexpr int plain_groups(int64_t n_seqs, int64_t total_q, int64_t max_seqlen_q,
+                           int32_t n_kv_heads, int g, int most, int cus) {
+  const BatchMix m = batch_mix(n_seqs, total_q, max_seqlen_q);
+  const auto queries = [&](int groups) -> int64_t { return 64 * groups / g; };  // of a tile
+  const auto tiles = [&](int groups) -> int64_t {
+    const int64_t qt = queries(groups);
+    return std::min(m.prompts * ((max_seqlen_q + qt - 1) / qt), m.prompt_rows / qt + m.prompts);
+  };
+  // workgroups, tiles counted by their size
+  const auto size = [&](int groups) -> int64_t {
+    return (tiles(groups) * groups / most + m.rows) * n_kv_heads;
+  };
+  int want = most;
+  if (g <= 64 && (size(1) <= cus || m.rows >= tiles(most))) {
+    want = 1;
+  } else if (most > 2) {
+    const bool used = 8 * most * queries(2) >= 7 * 2 * queries(most);
+    if (size(2) <= (used ? 16 : 2) * cus) want = 2;
+  }
+  // every sequence's tiles are launched as for the longest: more of them only while the empty
+  // ones are few, and no launch grows past what the largest tiles would take beyond that
+  const int64_t q = queries(want);
+  return n_seqs * ((max_seqlen_q + q - 1) / q) * n_kv_heads <= (1 << 16) ? want : most;
+}
+
+// Cost of one key step of a tile: its loads and the step's latency, and a share for each of
+// its four waves that has rows to compute. With a smaller base (1 of 5) a range of a sequence's
+// last, partial tile took up to twice the others' time: 1522 tokens in two chunks on 9000 (Hq 16,
+// Hk 8) 207 us, with 5 of 9 155; three chunks and 10 decode rows 70.5, 65.1.
+constexpr int kStepBase = 5;
+constexpr int kFullStep = kStepBase + 4;
+
+// Cost of a 16-key chunk of a decode row, in twentieths of a full tile's step: fewer workgroups
+// than the rows' share of the time alone would give them (5 and 3), since the memory serves them
+// at its full rate from half the chip's waves while the others compute. 48 rows with two
+// 512-token chunks, at 1, 2, 3, 4, 6: 116, 117, 126, 129, 160 us; 80 rows of 4k - 8k with one:
+// 333, 319, 316, 361; 60 fp8 rows with two: 88, 111, 119, 125.
+constexpr int row_cost(bool f8) { return f8 ? 1 : 2; }
+
+// The fewest workgroups of a KV head that the decode rows can have: each brings four waves, and
+// every group of `hp` KV heads and every one of its `ncg` column groups of query heads needs a
+// wave of its own (decode_stream.h).
+constexpr int row_ranges_least(int ncg, int hp) { return (ncg + 4 * hp - 1) / (4 * hp); }
+
+// Workgroups of each KV head for the decode rows and for the tiles.
+struct SplitShare {
+  int rows, tiles;
+};
+// n_ranges (more than row_ranges_least) workgroups of a KV head shared out by cost over `chunks`
+// chunks of decode rows and tiles of `tile_cost`: each kind of work that there is has at least
+// the fewest that do it, however little of it there is, since the rows are no tiles and only
+// their own workgroups compute them.
+constexpr SplitShare split_share(int n_ranges, int chunks, int tile_cost, bool f8, int ncg,
+                                 int hp) {
+  if (chunks <= 0) return SplitShare{0, n_ranges};
+  if (tile_cost <= 0) return SplitShare{n_ranges, 0};
+  const float cost = (float)chunks * ((float)(row_cost(f8) * kFullStep) / 20.f);
+  const int r = (int)((float)n_ranges * cost / (cost + (float)tile_cost) + 0.5f);
+  const int least = row_ranges_least(ncg, hp);
+  const int rows = r < least ? least : r < n_ranges - 1 ? r : n_ranges - 1;
+  return SplitShare{rows, n_ranges - rows};
+}
+
+// Whether a split launch's positions fit 32 bits with n_seqs sequences of up to `keys` keys (whose
+// lengths are 32 bits) and `tiles` tiles of theirs: the tiles' key steps by cost, of which a range's
+// end can lie as far past the last as a range is long, and the decode rows' chunks.
+constexpr bool split_fits(int64_t n_seqs, int64_t tiles, int64_t keys) {
+  constexpr int64_t most = 1000000000;
+  if (n_seqs > most || tiles > most) return false;  // the products below stay within 64 bits
+  if (keys > INT32_MAX) keys = INT32_MAX;
+  const int64_t steps = keys > 64 ? (keys + 63) / 64 : 1;
+  return tiles * steps * kFullStep <= most && n_seqs * ((keys + 15) / 16) <= most;
+}
+
+}  // namespace nkv

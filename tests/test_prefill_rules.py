@@ -1,5 +1,5 @@
-"""How a split launch shares its grid between tiles and decode rows (csrc/split_share.h, the
-code that the host plan and the kernels compile), compiled for the CPU: whatever the step's mix,
+"""The rules of the variable-length launches (csrc/prefill_rules.h, the code that the host and the
+kernels compile), compiled for the CPU. How a split launch shares its grid: whatever the step's mix,
 each kind of work that there is gets workgroups, since nothing else computes it, and the decode
 rows a wave for every group of KV heads and of query heads' columns."""
 import ctypes as C
@@ -13,10 +13,13 @@ from conftest import ROOT
 
 CSRC = os.path.join(ROOT, "nanokv-llm_amd", "csrc")
 SOURCE = r"""
-#include "split_share.h"
+#include "prefill_rules.h"
 extern "C" int share(int n, int chunks, int tiles, int f8, int ncg, int hp) {
   const nkv::SplitShare s = nkv::split_share(n, chunks, tiles, f8 != 0, ncg, hp);
   return s.rows * 65536 + s.tiles;
+}
+extern "C" int groups(int64_t n, int64_t total, int64_t max_q, int hk, int g, int most) {
+  return nkv::plain_groups(n, total, max_q, hk, g, most, 256);
 }
 extern "C" int fits(int64_t n_seqs, int64_t tiles, int64_t keys) {
   return nkv::split_fits(n_seqs, tiles, keys);
@@ -29,12 +32,13 @@ def lib(tmp_path_factory):
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ is not installed")
-    d = tmp_path_factory.mktemp("split_share")
-    src, so = d / "share.cpp", d / "share.so"
+    d = tmp_path_factory.mktemp("prefill_rules")
+    src, so = d / "rules.cpp", d / "rules.so"
     src.write_text(SOURCE)
     subprocess.run([gxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-fPIC", "-shared", "-I", CSRC,
                     str(src), "-o", str(so)], check=True)
     lib = C.CDLL(str(so))
+    lib.groups.argtypes = [C.c_int64] * 3 + [C.c_int] * 3
     lib.fits.argtypes = [C.c_int64] * 3
     return lib
 
@@ -86,3 +90,30 @@ def test_positions_of_a_stream_that_fits_stay_within_32_bits(lib):
     assert at_limit > 0
     # 2000 rows of a million keys (shared blocks): within; 200000: beyond
     assert lib.fits(2000, 2100, 1 << 20) == 1 and lib.fits(200000, 200100, 1 << 20) == 0
+
+
+@pytest.mark.parametrize("hk,g,mix,fastest", [
+    # prompt lengths, and the row groups per wave measured fastest (within 3%)
+    (8, 4, [333], 1), (8, 4, [1500], 1), (8, 4, [3000], 2), (8, 4, [2048] * 4, 2),
+    (8, 4, [1000] * 6, 2), (8, 4, [4096] * 16, 3), (8, 4, [1] * 80 + [300], 1),
+    (1, 24, [1300], 1), (1, 24, [2000], 2), (1, 24, [1000] * 6, 2), (4, 24, [600], 2),
+    (1, 33, [600], 1), (1, 33, [900], 2), (1, 33, [2000], 2), (1, 40, [3000], 2),
+    (1, 48, [600], 1), (1, 48, [900], 2), (1, 48, [1300], 2), (1, 48, [2000], 3),
+    (1, 48, [1000] * 6, 3), (2, 24, [2000], 2), (1, 72, [600], 2), (1, 72, [1300], 3),
+    (1, 96, [400], 2), (1, 96, [1300], 3), (1, 96, [1000] * 6, 3), (1, 128, [1500], 2),
+])
+@pytest.mark.parametrize("rows_known", [True, False])
+def test_plain_tile_size_is_the_measured_one(lib, hk, g, mix, fastest, rows_known):
+    # rows of q not known: every sequence's taken as the longest's
+    total = sum(mix) if rows_known or len(set(mix)) > 1 else -1
+    assert lib.groups(len(mix), total, max(mix), hk, g, 3) == fastest
+
+
+def test_plain_tile_size_is_one_that_holds_a_group(lib):
+    for most in (1, 2, 3):
+        for g in range(1, 129 if most > 1 else 65):
+            for n in (1, 5, 3000):
+                for max_q in (1, 2, 100, 5000, 10 ** 6):
+                    for total in (-1, n, n + max_q - 1, n * max_q):
+                        rg = lib.groups(n, total, max_q, 8, g, most)
+                        assert 1 <= rg <= most and 64 * rg >= g, (most, g, n, max_q, total)
