@@ -1,7 +1,7 @@
-// The rules by which the variable-length launches (prefill.hip) are chosen and share out their
-// work: a plain launch's tile size, and a split one's workgroups between the prompts' tiles and
-// the decode rows among them. Plain constexpr C++ that the host and the kernels compile, and a
-// test on the CPU.
+// Rules by which launches are chosen and share out their work: the variable-length attention's
+// (prefill.hip), a plain launch's tile size, and a split one's workgroups between the prompts'
+// tiles and the decode rows among them; and the waves that merge a decode row (paged_decode.hip).
+// Plain constexpr C++ that the host and the kernels compile, and a test on the CPU.
 #pragma once
 
 #include <stdint.h>
@@ -118,6 +118,25 @@ constexpr bool split_fits(int64_t n_seqs, int64_t tiles, int64_t keys) {
   if (keys > INT32_MAX) keys = INT32_MAX;
   const int64_t steps = keys > 64 ? (keys + 63) / 64 : 1;
   return tiles * steps * kFullStep <= most && n_seqs * ((keys + 15) / 16) <= most;
+}
+
+// Whether four waves merge the partials of a decode row instead of one: where a row may have more
+// than 24, its sequence's share of the `waves` waves of each KV head and column group, or as many as
+// a full table row makes (ranges of min_chunks of its max_chunks). One wave has 16 partials in
+// flight at once and eight more in another round trip; four pay for their own merge (split
+// and combine in a graph, one / four, us):
+//   1 sequence of 16000 (Hq 32, Hk 8; up to 127)           23.6 /  16.5
+//   3 of 1000 - 4000 (Hq 8, Hk 2; 87)                      16.2 /  11.4
+//   12 of 4000 - 16000 (Hq 16, Hk 8; 23)                   88.6 /  84.5
+//   100 of 250 - 1000 (Hq 16, Hk 1; 22)                    20.8 /  22.6
+//   100 of 1000 - 4000 (Hq 80, Hk 1; 6)                   125.1 / 138.9
+// Over 484 such shapes the line is nowhere slower than one wave alone, and 0.1% off the faster
+// choice on average, 4.9% at most; from 16 partials on and with the column groups left out, 87
+// of them were over 2% slower than one wave, up to 31%.
+constexpr bool combine_wide(int64_t batch, int64_t n_kv_heads, int64_t ncg, int64_t max_chunks,
+                            int64_t min_chunks, int64_t waves) {
+  const int64_t share = waves / (n_kv_heads * ncg) / batch + 2;
+  return std::min(share, (max_chunks + min_chunks - 1) / min_chunks + 1) > 24;
 }
 
 }  // namespace nkv

@@ -46,6 +46,7 @@
 //
 // head_dim D is 64, 128 or 256 (a template parameter of both kernels).
 #include "decode_stream.h"
+#include "launch_rules.h"
 
 #include <algorithm>
 #include <atomic>
@@ -333,14 +334,12 @@ static int decode_combine(const int32_t* context_lens, int32_t batch, int32_t n_
   const i32x4v_t* desc = static_cast<const i32x4v_t*>(workspace);
   const float* part = reinterpret_cast<const float*>(static_cast<const char*>(workspace) + desc_b);
   const dim3 grid((unsigned)(batch * n_q_heads));
-  // Four waves where a row may have more partials than one wave has loads in flight (16): at
-  // most one for every wave of its head group that the batch leaves to it, and no more than the
-  // table width lets a segment have (of a 16-bit pool: an fp8 one's ranges are no shorter).
+  // (the ranges of a 16-bit pool: an fp8 one's are no shorter)
   const int64_t max_chunks = decode_max_chunks(max_blocks_per_seq, block_size);
   const int64_t min_chunks =
       decode_min_chunks(max_chunks, decode_range_floor(batch, head_dim, false));
-  const int64_t shares = (int64_t)device_cus() * kWavesPerCU / n_kv_heads / batch + 2;
-  const bool wide = std::min(shares, (max_chunks + min_chunks - 1) / min_chunks + 1) > 16;
+  const bool wide = combine_wide(batch, n_kv_heads, ncg, max_chunks, min_chunks,
+                                 (int64_t)device_cus() * kWavesPerCU);
 #define NKV_COMBINE_LAUNCH_W(D, W)                                                             \
   hipLaunchKernelGGL((paged_decode_combine_kernel<D, H16, W>), grid, dim3(64 * W), 0,          \
                      as_stream(stream), context_lens, n_q_heads, n_kv_heads, ncg, part, desc,  \

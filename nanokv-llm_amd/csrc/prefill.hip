@@ -44,7 +44,7 @@
 //    second kernel merges the cut tiles; decode rows (one new token) are streamed by waves of
 //    workgroups of their own, as the decode kernel does.
 #include "decode_stream.h"
-#include "prefill_rules.h"
+#include "launch_rules.h"
 
 #include <algorithm>
 #include <type_traits>

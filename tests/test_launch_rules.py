@@ -1,4 +1,4 @@
-"""The rules of the variable-length launches (csrc/prefill_rules.h, the code that the host and the
+"""The rules by which launches are chosen (csrc/launch_rules.h, the code that the host and the
 kernels compile), compiled for the CPU. How a split launch shares its grid: whatever the step's mix,
 each kind of work that there is gets workgroups, since nothing else computes it, and the decode
 rows a wave for every group of KV heads and of query heads' columns."""
@@ -13,13 +13,16 @@ from conftest import ROOT
 
 CSRC = os.path.join(ROOT, "nanokv-llm_amd", "csrc")
 SOURCE = r"""
-#include "prefill_rules.h"
+#include "launch_rules.h"
 extern "C" int share(int n, int chunks, int tiles, int f8, int ncg, int hp) {
   const nkv::SplitShare s = nkv::split_share(n, chunks, tiles, f8 != 0, ncg, hp);
   return s.rows * 65536 + s.tiles;
 }
 extern "C" int groups(int64_t n, int64_t total, int64_t max_q, int hk, int g, int most) {
   return nkv::plain_groups(n, total, max_q, hk, g, most, 256);
+}
+extern "C" int wide(int64_t batch, int64_t hk, int64_t ncg, int64_t max_c, int64_t min_c) {
+  return nkv::combine_wide(batch, hk, ncg, max_c, min_c, 2048);
 }
 extern "C" int fits(int64_t n_seqs, int64_t tiles, int64_t keys) {
   return nkv::split_fits(n_seqs, tiles, keys);
@@ -32,13 +35,14 @@ def lib(tmp_path_factory):
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ is not installed")
-    d = tmp_path_factory.mktemp("prefill_rules")
+    d = tmp_path_factory.mktemp("launch_rules")
     src, so = d / "rules.cpp", d / "rules.so"
     src.write_text(SOURCE)
     subprocess.run([gxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-fPIC", "-shared", "-I", CSRC,
                     str(src), "-o", str(so)], check=True)
     lib = C.CDLL(str(so))
     lib.groups.argtypes = [C.c_int64] * 3 + [C.c_int] * 3
+    lib.wide.argtypes = [C.c_int64] * 5
     lib.fits.argtypes = [C.c_int64] * 3
     return lib
 
@@ -117,3 +121,19 @@ def test_plain_tile_size_is_one_that_holds_a_group(lib):
                     for total in (-1, n, n + max_q - 1, n * max_q):
                         rg = lib.groups(n, total, max_q, 8, g, most)
                         assert 1 <= rg <= most and 64 * rg >= g, (most, g, n, max_q, total)
+
+
+@pytest.mark.parametrize("hq,hk,batch,longest,wide", [
+    # the waves a row's merge measured fastest with (table rows of 256-token blocks)
+    (32, 8, 1, 16000, True), (32, 8, 5, 16000, True), (8, 2, 3, 4000, True),
+    (64, 1, 1, 16000, True), (64, 2, 12, 4000, True), (80, 1, 8, 4000, True),
+    (16, 8, 5, 1000, False), (16, 1, 100, 1000, False), (64, 2, 32, 1000, False),
+    (64, 1, 64, 4000, False), (64, 1, 100, 4000, False), (64, 2, 64, 4000, False),
+    (32, 1, 100, 4000, False), (80, 1, 64, 4000, False), (80, 1, 100, 4000, False),
+    (32, 8, 64, 8192, False),
+])
+def test_merge_waves_are_the_measured_ones(lib, hq, hk, batch, longest, wide):
+    g = hq // hk
+    chunks = -(-longest // 256) * 16
+    assert lib.wide(batch, hk, -(-g // 16) if g > 16 else 1, chunks,
+                    max(3 if batch > 2 else 4, -(-chunks // 128))) == wide
