@@ -214,6 +214,15 @@ def varlen_prefill_workspace(q: torch.Tensor, k: torch.Tensor, n_seqs: int, max_
     return torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
 
 
+def _step_workspace(q, k_cache, n_seqs, context):
+    """The split launch's workspace for a paged step, or None (the plain launch): also where the
+    context leaves the longest key length out, which only this choice goes by."""
+    longest = context.max_seqlen_k
+    if longest is None or longest <= _SPLIT_MIN_KEYS:
+        return None
+    return varlen_prefill_workspace(q, k_cache, n_seqs, context.max_seqlen_q, longest)
+
+
 def varlen_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                    cu_seqlens_q: torch.Tensor, cu_seqlens_k: torch.Tensor, max_seqlen_q: int,
                    scale: float, block_tables: torch.Tensor | None = None,
@@ -436,10 +445,7 @@ class Attention(nn.Module):
             if n_seqs < 0 or cu_k.numel() != n_seqs + 1:
                 return None
             max_q = int(context.max_seqlen_q)
-            workspace = None
-            if context.max_seqlen_k > _SPLIT_MIN_KEYS:
-                workspace = varlen_prefill_workspace(q, k_cache, n_seqs, max_q,
-                                                     context.max_seqlen_k)
+            workspace = _step_workspace(q, k_cache, n_seqs, context)
         out = q.new_empty(qs)
         kv_type = _lib.NKV_KV_FP8 if ct is _FP8 else \
             _lib.NKV_KV_F16 if dt is _F16 else _lib.NKV_KV_BF16
@@ -494,11 +500,8 @@ class Attention(nn.Module):
 
         if not context.use_decode_kernel:
             if context.block_tables is not None:  # K/V read back from the paged cache
-                workspace = None
-                if context.max_seqlen_k > _SPLIT_MIN_KEYS:
-                    workspace = varlen_prefill_workspace(
-                        q, k_cache, context.cu_seqlens_q.numel() - 1, context.max_seqlen_q,
-                        context.max_seqlen_k)
+                workspace = _step_workspace(q, k_cache, context.cu_seqlens_q.numel() - 1,
+                                            context)
                 return varlen_prefill(q, k_cache, v_cache, context.cu_seqlens_q,
                                       context.cu_seqlens_k, context.max_seqlen_q, self.scale,
                                       block_tables=context.block_tables,

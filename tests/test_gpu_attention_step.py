@@ -100,6 +100,14 @@ def test_other_forms_keep_the_separate_calls_answers(nkv, dev):
     assert torch.equal(out, ref)
 
 
+@pytest.mark.gpu
+def test_no_longest_key_length_takes_the_plain_launch(nkv, dev):
+    layer, args, ctx = _step(dev, "bf16", False, False)
+    some = _run(nkv, layer, args, ctx[:4] + (0,) + ctx[5:])
+    none = _run(nkv, layer, args, ctx[:4] + (None,) + ctx[5:])
+    assert all(torch.equal(a, b) for a, b in zip(some, none))
+
+
 def test_the_call_checks_its_arguments_on_the_host():
     lib = L.lib()
     pack = attention._ATTENTION_ARGS.pack

@@ -128,3 +128,22 @@ def test_shared_workspace_kept_only_when_captured(monkeypatch):
     assert len(attn._RETIRED_WS) == 1 and attn._RETIRED_WS[0] is w2 and w3 is not w2
     assert attn.release_retired_decode_workspaces() == 1 and attn._RETIRED_WS == []
     del w1
+
+
+def test_attention_takes_a_context_without_the_longest_key_length(monkeypatch):
+    """max_seqlen_k is only a hint for the choice of launch: None takes the plain one."""
+    from types import SimpleNamespace
+    calls = []
+    monkeypatch.setattr(attn, "varlen_prefill", lambda *a, **kw: calls.append(kw) or a[0])
+    layer = attn.Attention(8, 128, 0.1, 2, SimpleNamespace(kv_compress_enabled=False), 1)
+    layer.k_cache = layer.v_cache = torch.zeros(4, 256, 2, 128, dtype=BF)
+    q = torch.zeros(3, 8, 128, dtype=BF)
+    cu = torch.tensor([0, 3], dtype=I32)
+    for longest in (None, 0, 700):
+        ctx = SimpleNamespace(use_decode_kernel=False, is_compress_step=False, cu_seqlens_q=cu,
+                              cu_seqlens_k=cu, max_seqlen_q=3, max_seqlen_k=longest,
+                              slot_mapping=None, block_tables=torch.zeros(1, 4, dtype=I32))
+        monkeypatch.setattr(attn, "get_context", lambda: ctx)
+        assert layer(q, None, None, 0, kv_stored=True) is q
+        assert calls[-1]["workspace"] is None
+    assert len(calls) == 3
