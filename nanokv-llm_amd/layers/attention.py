@@ -205,13 +205,18 @@ def varlen_prefill_workspace(q: torch.Tensor, k: torch.Tensor, n_seqs: int, max_
                              max_seqlen_k: int) -> torch.Tensor | None:
     """The workspace for splitting varlen_prefill's keys where that is the faster way (a few
     query tiles, or a long context among short ones: the longest sequence would otherwise hold
-    the call up), else None. Sized by the chip, not by the lengths."""
+    the call up), else None. Sized by the chip, not by the lengths (121 MB at 32 query heads of
+    128 over a bf16 pool); None too where the device has no such memory left, since the plain
+    launch needs none."""
     t = _lib.NKV_KV_FP8 if k.dtype == torch.float8_e4m3fn else \
         _lib.NKV_KV_F16 if k.dtype == torch.float16 else _lib.NKV_KV_BF16
     nbytes = _lib.lib().nkv_prefill_split_plan(n_seqs, q.size(0), int(max_seqlen_q),
                                                int(max_seqlen_k), q.size(1), k.size(-2),
                                                q.size(2), t)
-    return torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+    except torch.OutOfMemoryError:
+        return None
 
 
 def _step_workspace(q, k_cache, n_seqs, context):
@@ -436,7 +441,7 @@ class Attention(nn.Module):
         if decode:
             if n_seqs < N or lens.numel() < N:
                 return None
-            n_seqs, max_q = N, 0
+            n_seqs, max_q, out = N, 0, q.new_empty(qs)
             if torch.cuda.is_current_stream_capturing():
                 workspace = self._workspace(q, bt)
             else:
@@ -444,9 +449,8 @@ class Attention(nn.Module):
         else:
             if n_seqs < 0 or cu_k.numel() != n_seqs + 1:
                 return None
-            max_q = int(context.max_seqlen_q)
+            max_q, out = int(context.max_seqlen_q), q.new_empty(qs)  # before the workspace
             workspace = _step_workspace(q, k_cache, n_seqs, context)
-        out = q.new_empty(qs)
         kv_type = _lib.NKV_KV_FP8 if ct is _FP8 else \
             _lib.NKV_KV_F16 if dt is _F16 else _lib.NKV_KV_BF16
         lib = _lib.lib()
@@ -500,11 +504,12 @@ class Attention(nn.Module):
 
         if not context.use_decode_kernel:
             if context.block_tables is not None:  # K/V read back from the paged cache
+                out = torch.empty(q.shape, dtype=q.dtype, device=q.device)  # before the workspace
                 workspace = _step_workspace(q, k_cache, context.cu_seqlens_q.numel() - 1,
                                             context)
                 return varlen_prefill(q, k_cache, v_cache, context.cu_seqlens_q,
                                       context.cu_seqlens_k, context.max_seqlen_q, self.scale,
-                                      block_tables=context.block_tables,
+                                      block_tables=context.block_tables, out=out,
                                       max_seqlen_k=context.max_seqlen_k, k_scale=self.k_scale,
                                       v_scale=self.v_scale, workspace=workspace)
             return varlen_prefill(q, k, v, context.cu_seqlens_q, context.cu_seqlens_k,

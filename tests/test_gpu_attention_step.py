@@ -108,6 +108,34 @@ def test_no_longest_key_length_takes_the_plain_launch(nkv, dev):
     assert all(torch.equal(a, b) for a, b in zip(some, none))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("kv_stored", [False, True])
+def test_a_full_card_runs_the_plain_launch(nkv, dev, kv_stored):
+    """Torch's allocator limited to what a step that splits needs without its workspace."""
+    g = torch.Generator().manual_seed(4)
+    lens = torch.tensor([0, 130], dtype=torch.int32), torch.tensor([0, 9000], dtype=torch.int32)
+    q, k, v = (torch.randn(130, h, 128, generator=g).bfloat16().to(dev) for h in (32, 8, 8))
+    layer = attention.Attention(32, 128, 128 ** -0.5, 8, NO_COMPRESSION, 1)
+    layer.k_cache, layer.v_cache = torch.randn(2, 36, 256, 8, 128, generator=g).bfloat16().to(dev)
+    bt = torch.arange(36, dtype=torch.int32).view(1, 36).to(dev)
+    slots = torch.arange(8870, 9000, dtype=torch.int32).to(dev)
+    cu_q, cu_k = (x.to(dev) for x in lens)
+    assert attention.varlen_prefill_workspace(q, layer.k_cache, 1, 130, 9000).numel() > 64 << 20
+    nkv.set_context(False, cu_q, cu_k, 130, 9000, slots, None, bt)
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(dev).total_memory
+    torch.cuda.set_per_process_memory_fraction(
+        (torch.cuda.memory_reserved(dev) + (32 << 20)) / total, dev)
+    try:
+        out = layer(q, k, v, 0, kv_stored=kv_stored)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+        nkv.reset_context()
+    plain = nkv.varlen_prefill(q, layer.k_cache, layer.v_cache, cu_q, cu_k, 130, 128 ** -0.5,
+                               block_tables=bt)
+    assert torch.equal(out, plain)
+
+
 def test_the_call_checks_its_arguments_on_the_host():
     lib = L.lib()
     pack = attention._ATTENTION_ARGS.pack

@@ -147,3 +147,34 @@ def test_attention_takes_a_context_without_the_longest_key_length(monkeypatch):
         assert layer(q, None, None, 0, kv_stored=True) is q
         assert calls[-1]["workspace"] is None
     assert len(calls) == 3
+
+
+def test_no_memory_for_the_split_launch_takes_the_plain_one(monkeypatch):
+    """The split launch's workspace is a help, not a need: a card that the pool fills runs the
+    step in the memory of its output, which is taken first."""
+    from types import SimpleNamespace
+    q = torch.zeros(512, 32, 128, dtype=BF)
+    kc = torch.zeros(2, 256, 8, 128, dtype=BF)
+    assert attn.varlen_prefill_workspace(q, kc, 1, 512, 12800).numel() > 1 << 26
+    order = []
+
+    def empty(*size, **kw):
+        order.append(kw["dtype"])
+        if kw["dtype"] is torch.uint8:
+            raise torch.OutOfMemoryError("no memory")
+        return torch.zeros(*size, **kw)
+    monkeypatch.setattr(torch, "empty", empty)
+    assert attn.varlen_prefill_workspace(q, kc, 1, 512, 12800) is None
+    calls = []
+    monkeypatch.setattr(attn, "varlen_prefill", lambda *a, **kw: calls.append(kw) or kw["out"])
+    layer = attn.Attention(32, 128, 0.1, 8, SimpleNamespace(kv_compress_enabled=False), 1)
+    layer.k_cache = layer.v_cache = kc
+    cu = torch.tensor([0, 512], dtype=I32)
+    ctx = SimpleNamespace(use_decode_kernel=False, is_compress_step=False, cu_seqlens_q=cu,
+                          cu_seqlens_k=cu, max_seqlen_q=512, max_seqlen_k=12800,
+                          slot_mapping=None, block_tables=torch.zeros(1, 50, dtype=I32))
+    monkeypatch.setattr(attn, "get_context", lambda: ctx)
+    order.clear()
+    out = layer(q, None, None, 0, kv_stored=True)
+    assert order == [BF, torch.uint8] and out.shape == q.shape and out.dtype == q.dtype
+    assert calls[0]["workspace"] is None
