@@ -78,12 +78,21 @@ constexpr int plain_groups(int64_t n_seqs, int64_t total_q, int64_t max_seqlen_q
 constexpr int kStepBase = 5;
 constexpr int kFullStep = kStepBase + 4;
 
-// Cost of a 16-key chunk of a decode row, in twentieths of a full tile's step: fewer workgroups
-// than the rows' share of the time alone would give them (5 and 3), since the memory serves them
-// at its full rate from half the chip's waves while the others compute. 48 rows with two
-// 512-token chunks, at 1, 2, 3, 4, 6: 116, 117, 126, 129, 160 us; 80 rows of 4k - 8k with one:
-// 333, 319, 316, 361; 60 fp8 rows with two: 88, 111, 119, 125.
-constexpr int row_cost(bool f8) { return f8 ? 1 : 2; }
+// Cost of a 16-key chunk of a decode row for one KV head, a full tile's step being kFullStep: fewer
+// workgroups than the rows' share of the time alone would give them (5 / 20 and 3 / 20 of a step in
+// bf16 and fp8 at head_dim 128), since the memory serves them at its full rate from half the
+// chip's waves while the others compute. 48 rows with two 512-token chunks, at 1, 2, 3, 4, 6
+// twentieths: 116, 117, 126, 129, 160 us; 80 rows of 4k - 8k with one: 333, 319, 316, 361; 60 fp8
+// rows with two: 88, 111, 119, 125. At head_dim 256 a chunk is twice the bytes beside a step of a
+// third of the rows, and each of `ncg` column groups streams it. Times over the best share's,
+// geometric mean (worst), of random steps: 2 (bf16) and 1 (fp8) twentieths everywhere / as here
+//   head_dim 256: 38 steps 1.10 (1.5) / 1.02 (1.1); fp8, 19 steps 1.30 (2.0) / 1.05 (1.3)
+//   head_dim 128, four groups: 11 steps 1.18 (1.7) / 1.04 (1.1); fp8, 4 steps 1.36 / 1.17
+//   head_dim 256, four groups: 6 steps 1.96 (2.7) / 1.03 (1.1)
+constexpr float row_cost(int head_dim, bool f8, int ncg) {
+  const int twentieths = head_dim == 256 ? (f8 ? 3 : 4) : (f8 ? 1 : 2);
+  return (float)(twentieths * ncg * kFullStep) / 20.f;
+}
 
 // The fewest workgroups of a KV head that the decode rows can have: each brings four waves, and
 // every group of `hp` KV heads and every one of its `ncg` column groups of query heads needs a
@@ -98,11 +107,11 @@ struct SplitShare {
 // chunks of decode rows and tiles of `tile_cost`: each kind of work that there is has at least
 // the fewest that do it, however little of it there is, since the rows are no tiles and only
 // their own workgroups compute them.
-constexpr SplitShare split_share(int n_ranges, int chunks, int tile_cost, bool f8, int ncg,
-                                 int hp) {
+constexpr SplitShare split_share(int n_ranges, int chunks, float chunk_cost, int tile_cost,
+                                 int ncg, int hp) {
   if (chunks <= 0) return SplitShare{0, n_ranges};
   if (tile_cost <= 0) return SplitShare{n_ranges, 0};
-  const float cost = (float)chunks * ((float)(row_cost(f8) * kFullStep) / 20.f);
+  const float cost = (float)chunks * chunk_cost;
   const int r = (int)((float)n_ranges * cost / (cost + (float)tile_cost) + 0.5f);
   const int least = row_ranges_least(ncg, hp);
   const int rows = r < least ? least : r < n_ranges - 1 ? r : n_ranges - 1;

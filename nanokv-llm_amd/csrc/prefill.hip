@@ -114,6 +114,7 @@ struct SplitArgs {
   i32x4v_t* row_desc;
   float* row_part;
   int32_t max_tokens;  // keys that a table row holds
+  float chunk_cost;    // row_cost
 };
 constexpr int kSnap = 2;  // a range never cuts a unit within this many steps of its ends
 
@@ -190,8 +191,9 @@ __device__ __forceinline__ bool split_begin(const SplitArgs& sa,
   int n_ranges = (int)gridDim.x / Hk;  // of each KV head
   c.row_groups = 0;
   if constexpr (ROWS) {
-    const SplitShare share = split_share(
-        n_ranges, __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63), T, F8, sa.ncg, HP);
+    const SplitShare share =
+        split_share(n_ranges, __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63),
+                    sa.chunk_cost, T, sa.ncg, HP);
     n_ranges = share.tiles;
     c.row_groups = share.rows * Hk;
     if ((int)blockIdx.x < c.row_groups) return false;
@@ -1123,6 +1125,7 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
         (int64_t)max_blocks * block_size < (1ll << 30) &&
         (int64_t)block_size * k_row_stride * kEl < (1ll << 31)) {
       sa.max_tokens = max_blocks * block_size;
+      sa.chunk_cost = row_cost(head_dim, F8, sa.ncg);
       row_heads = prefill_row_heads<F8>(n_kv_heads, g, head_dim);
       if (prefill_ranges(n_kv_heads, head_dim) <= row_ranges_least(sa.ncg, row_heads))
         row_heads = 0;

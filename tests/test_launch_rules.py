@@ -14,8 +14,9 @@ from conftest import ROOT
 CSRC = os.path.join(ROOT, "nanokv-llm_amd", "csrc")
 SOURCE = r"""
 #include "launch_rules.h"
-extern "C" int share(int n, int chunks, int tiles, int f8, int ncg, int hp) {
-  const nkv::SplitShare s = nkv::split_share(n, chunks, tiles, f8 != 0, ncg, hp);
+extern "C" int share(int n, int chunks, int tiles, int dim, int f8, int ncg, int hp) {
+  const nkv::SplitShare s =
+      nkv::split_share(n, chunks, nkv::row_cost(dim, f8 != 0, ncg), tiles, ncg, hp);
   return s.rows * 65536 + s.tiles;
 }
 extern "C" int groups(int64_t n, int64_t total, int64_t max_q, int hk, int g, int most) {
@@ -68,7 +69,7 @@ def test_every_kind_of_work_gets_workgroups(lib, f8):
             for tiles in (0, 5, 9, 90, 7000, 10 ** 6, 10 ** 9):
                 if chunks == tiles == 0:
                     continue
-                s = lib.share(n, chunks, tiles, f8, ncg, hp)
+                s = lib.share(n, chunks, tiles, 128, f8, ncg, hp)
                 rows, left = s >> 16, s & 0xffff
                 at = (n, hk, ncg, hp, chunks, tiles, rows, left)
                 assert rows + left == n, at
@@ -137,3 +138,17 @@ def test_merge_waves_are_the_measured_ones(lib, hq, hk, batch, longest, wide):
     chunks = -(-longest // 256) * 16
     assert lib.wide(batch, hk, -(-g // 16) if g > 16 else 1, chunks,
                     max(3 if batch > 2 else 4, -(-chunks // 128))) == wide
+
+
+@pytest.mark.parametrize("dim,f8,ncg,best", [
+    # the multiples of 2 (bf16) and 1 (fp8) twentieths of a step a chunk whose shares were measured
+    # within 10% of the best share on average
+    (128, 0, 1, (0.5, 2)), (128, 1, 1, (0.75, 3)), (64, 0, 1, (0.5, 2)), (64, 1, 1, (0.75, 2)),
+    (256, 0, 1, (1, 2)), (256, 1, 1, (2, 3)), (128, 0, 2, (1, 3)), (128, 0, 4, (1.5, 6)),
+    (128, 1, 2, (1.5, 6)), (256, 0, 2, (4, 6)), (256, 0, 4, (6, 10)), (256, 1, 4, (10, 16)),
+])
+def test_decode_rows_share_is_near_the_measured_best(lib, dim, f8, ncg, best):
+    n, chunks, tiles = 512, 2000, 40000
+    rows = lib.share(n, chunks, tiles, dim, f8, ncg, 1) >> 16
+    lo, hi = (n * x / (x + tiles) for x in (chunks * m * (0.45 if f8 else 0.9) for m in best))
+    assert lo - 1 <= rows <= hi + 1
