@@ -119,8 +119,8 @@ constexpr SplitShare split_share(int n_ranges, int chunks, float chunk_cost, int
 }
 
 // Whether a split launch's positions fit 32 bits with n_seqs sequences of up to `keys` keys (whose
-// lengths are 32 bits) and `tiles` tiles of theirs: the tiles' key steps by cost, of which a range's
-// end can lie as far past the last as a range is long, and the decode rows' chunks.
+// lengths are 32 bits) and `tiles` tiles of theirs: the tiles' key steps by cost, of which a
+// range's end can lie as far past the last as a range is long, and the decode rows' chunks.
 constexpr bool split_fits(int64_t n_seqs, int64_t tiles, int64_t keys) {
   constexpr int64_t most = 1000000000;
   if (n_seqs > most || tiles > most) return false;  // the products below stay within 64 bits
@@ -130,8 +130,8 @@ constexpr bool split_fits(int64_t n_seqs, int64_t tiles, int64_t keys) {
 }
 
 // Whether four waves merge the partials of a decode row instead of one: where a row may have more
-// than 24, its sequence's share of the `waves` waves of each KV head and column group, or as many as
-// a full table row makes (ranges of min_chunks of its max_chunks). One wave has 16 partials in
+// than 24, its sequence's share of the `waves` waves of each KV head and column group, or as many
+// as a full table row makes (ranges of min_chunks of its max_chunks). One wave has 16 partials in
 // flight at once and eight more in another round trip; four pay for their own merge (split
 // and combine in a graph, one / four, us):
 //   1 sequence of 16000 (Hq 32, Hk 8; up to 127)           23.6 /  16.5

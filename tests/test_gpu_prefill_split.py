@@ -291,6 +291,13 @@ def test_plain_tile_sizes_match_the_oracle(nkv, dev, kind, Hq, Hk, D, n):
     assert bool(torch.isfinite(out.float()).all())
 
 
+# (sequences, rows of q, longest new and key lengths, Hq, Hk, head_dim, kv_type): split launches
+# measured at 0.55 of the plain one's time or less
+SPLIT_FASTER = [(40, 135, 96, 2203, 32, 8, 256, 0), (1, 10, 10, 1748, 8, 8, 256, 2),
+                (40, 54, 15, 6000, 128, 2, 128, 2), (1, 5, 5, 3255, 48, 1, 256, 0),
+                (2, 95, 85, 11968, 28, 4, 256, 2), (40, 237, 193, 727, 8, 8, 256, 0)]
+
+
 def test_split_plan_and_arguments_on_the_host():
     """The rule, and what the entry point refuses, without a GPU."""
     lib = L.lib()
@@ -306,6 +313,17 @@ def test_split_plan_and_arguments_on_the_host():
     assert plan(1, 512, 512, 0, 32, 8, 128, L.NKV_KV_BF16) == 0
     assert plan(0, 0, 0, 0, 32, 8, 128, L.NKV_KV_BF16) == 0
     assert plan(1, 512, 512, 12800, 30, 8, 128, L.NKV_KV_BF16) == 0
+    # steps that the plain launch was measured faster for: tiles of head_dim 256, and rows that
+    # several column groups stream; and those where the split one was still
+    bf16 = L.NKV_KV_BF16
+    assert plan(16, 1923, 560, 853, 16, 16, 256, bf16) == 0  # plain 55 us, split 73
+    assert plan(5, 3668, 1824, 6770, 16, 16, 256, bf16) == 0  # 476, 606
+    assert plan(80, 81, 2, 2132, 128, 2, 256, bf16) == 0  # 81, 129
+    assert plan(150, 217, 68, 2462, 96, 1, 128, bf16) == 0  # 96, 112
+    assert plan(150, 158, 9, 4398, 128, 2, 128, bf16) == 0  # 122, 182
+    assert plan(40, 995, 597, 6000, 28, 4, 256, bf16) > 0  # within 20%
+    for args in SPLIT_FASTER:
+        assert plan(*args) > 0, args
     # positions in 32 bits: 200 rows of a million keys, not 2000 of eight
     assert plan(200, 711, 512, 1 << 20, 32, 8, 128, L.NKV_KV_BF16) == size(200)
     assert plan(2000, 2511, 512, 1 << 23, 32, 8, 128, L.NKV_KV_BF16) == 0
