@@ -27,17 +27,28 @@ constexpr BatchMix batch_mix(int64_t n_seqs, int64_t total_q, int64_t max_seqlen
   return m;
 }
 
+// Tiles of qt queries a sequence in a plain launch's grid, enough for the longest: with more than one
+// sequence an odd number. Most sequences of a mixed step have one tile (a decode row), every
+// plain_tiles-th workgroup of a KV head, and workgroups go to XCDs and CUs in turn: a stride with
+// powers of two in it leaves the work to a few of them. 250 rows of up to 500 keys and a prompt
+// (Hq 32, Hk 8, 64 rows a tile, even / odd, us): of 120 tokens (8, 9 tiles) 199 / 78, of 500 (32,
+// 33) 215 / 100; Hq 8, Hk 2: 145 / 31.
+constexpr int64_t plain_tiles(int64_t n_seqs, int64_t max_seqlen_q, int64_t qt) {
+  const int64_t tiles = (max_seqlen_q + qt - 1) / qt;
+  return n_seqs > 1 ? tiles | 1 : tiles;
+}
+
 // Row groups per wave of a plain launch, up to `most` (every number gives the same bits). More rows
 // a tile need fewer reads of K and V from LDS per MFMA, fewer leave more workgroups to overlap, and
 // a workgroup's key step takes 1.15 us with one, 1.26 with two, 1.75 with three while the chip is
 // not full. Measured (Hq 32, Hk 8; 1 / 2 / 3 groups, us; workgroups as with three):
-//   a prompt of 333 (56 workgroups)     11.2 /  14.4 /  20.2
-//   of 1500 (256)                       33.4 /  38.0 /  51.6
-//   of 3000 (504)                       95.5 /  80.2 /  98.3
-//   four chunks of 2048 on 6000 (1376)  1053 /   809 /   841
-//   16 prompts up to 1500 (3144)         305 /   229 /   241
-//   16 prompts up to 4096 (8472)        1682 /  1315 /  1294
-//   80 decode rows, a prompt of 300      34.3 /  51.0 /  46.9 (a row's tile is a row)
+//   a prompt of 333 (56 workgroups)     10.1 /  13.2 /  18.9
+//   of 1500 (256)                       34.1 /  38.1 /  50.6
+//   of 3000 (504)                      100.0 /  81.8 /  99.4
+//   four chunks of 2048 on 6000 (1376)  1059 /   816 /   847
+//   16 prompts up to 1500 (4224)         206 /   159 /   170
+//   16 prompts up to 4096 (11136)       1206 /   933 /   925
+//   250 decode rows, a prompt of 60      35.3 /  41.4 /  52.9 (a row's tile is a row)
 // Large GQA groups g leave a part of a tile's rows unused, more of a small tile's (a group of 48
 // fills 192 rows, 96 of 128): the lines lie at the tiles that there are of each size, and on a
 // full chip two groups need 7/8 of the use that `most` makes of its rows (1 / 2 / 3, us):
@@ -65,10 +76,15 @@ constexpr int plain_groups(int64_t n_seqs, int64_t total_q, int64_t max_seqlen_q
     const bool used = 8 * most * queries(2) >= 7 * 2 * queries(most);
     if (size(2) <= (used ? 16 : 2) * cus) want = 2;
   }
-  // every sequence's tiles are launched as for the longest: more of them only while the empty
-  // ones are few, and no launch grows past what the largest tiles would take beyond that
-  const int64_t q = queries(want);
-  return n_seqs * ((max_seqlen_q + q - 1) / q) * n_kv_heads <= (1 << 16) ? want : most;
+  // Every sequence's tiles are launched as for the longest, and each empty workgroup takes its turn:
+  // the smaller sizes only while a launch stays small. 120 rows and 4 prompts of 500 (Hq 64, Hk 8;
+  // 64480, 32736, 20832 workgroups): 89 / 69 / 70 us.
+  const auto launched = [&](int groups) -> int64_t {
+    return n_seqs * plain_tiles(n_seqs, max_seqlen_q, queries(groups)) * n_kv_heads;
+  };
+  if (want == 1 && launched(1) > 24576) want = std::min(most, 2);
+  if (want == 2 && launched(2) > 49152) want = most;
+  return want;
 }
 
 // Cost of one key step of a tile: its loads and the step's latency, and a share for each of

@@ -1100,9 +1100,10 @@ static int prefill_launch(const void* q, int64_t q_row_stride, const void* k_cac
                                           prefill_row_groups(head_dim, F8), device_cus());
   const int tile_rows = 64 * groups;
   const int qt = tile_rows / g;
-  const int n_tiles = (max_seqlen_q + qt - 1) / qt;
+  const int64_t tiles = plain_tiles(n_seqs, max_seqlen_q, qt);
   const float sl2 = scale * k_scale * kLog2e;
-  int64_t grid = (int64_t)n_seqs * n_tiles * n_kv_heads;
+  int64_t grid = n_seqs * tiles * n_kv_heads;
+  const int32_t n_tiles = (int32_t)tiles;
   int64_t merge_grid = 0;
   int row_heads = 0;
   SplitArgs sa = {};

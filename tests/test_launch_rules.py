@@ -22,6 +22,9 @@ extern "C" int share(int n, int chunks, int tiles, int dim, int f8, int ncg, int
 extern "C" int groups(int64_t n, int64_t total, int64_t max_q, int hk, int g, int most) {
   return nkv::plain_groups(n, total, max_q, hk, g, most, 256);
 }
+extern "C" int64_t tiles(int64_t n, int64_t max_q, int64_t qt) {
+  return nkv::plain_tiles(n, max_q, qt);
+}
 extern "C" int wide(int64_t batch, int64_t hk, int64_t ncg, int64_t max_c, int64_t min_c) {
   return nkv::combine_wide(batch, hk, ncg, max_c, min_c, 2048);
 }
@@ -43,6 +46,7 @@ def lib(tmp_path_factory):
                     str(src), "-o", str(so)], check=True)
     lib = C.CDLL(str(so))
     lib.groups.argtypes = [C.c_int64] * 3 + [C.c_int] * 3
+    lib.tiles.argtypes, lib.tiles.restype = [C.c_int64] * 3, C.c_int64
     lib.wide.argtypes = [C.c_int64] * 5
     lib.fits.argtypes = [C.c_int64] * 3
     return lib
@@ -101,6 +105,8 @@ def test_positions_of_a_stream_that_fits_stay_within_32_bits(lib):
     # prompt lengths, and the row groups per wave measured fastest (within 3%)
     (8, 4, [333], 1), (8, 4, [1500], 1), (8, 4, [3000], 2), (8, 4, [2048] * 4, 2),
     (8, 4, [1000] * 6, 2), (8, 4, [4096] * 16, 3), (8, 4, [1] * 80 + [300], 1),
+    (8, 4, [1] * 250 + [120], 1), (8, 4, [1] * 250 + [500], 2), (8, 8, [1] * 120 + [500] * 4, 2),
+    (8, 8, [1] * 250 + [300], 2), (8, 8, [1] * 250 + [500] * 4, 3), (2, 4, [1] * 250 + [500], 1),
     (1, 24, [1300], 1), (1, 24, [2000], 2), (1, 24, [1000] * 6, 2), (4, 24, [600], 2),
     (1, 33, [600], 1), (1, 33, [900], 2), (1, 33, [2000], 2), (1, 40, [3000], 2),
     (1, 48, [600], 1), (1, 48, [900], 2), (1, 48, [1300], 2), (1, 48, [2000], 3),
@@ -152,3 +158,13 @@ def test_decode_rows_share_is_near_the_measured_best(lib, dim, f8, ncg, best):
     rows = lib.share(n, chunks, tiles, dim, f8, ncg, 1) >> 16
     lo, hi = (n * x / (x + tiles) for x in (chunks * m * (0.45 if f8 else 0.9) for m in best))
     assert lo - 1 <= rows <= hi + 1
+
+
+def test_tiles_of_a_grid_cover_the_longest_sequence_at_an_odd_stride(lib):
+    for qt in (1, 2, 16, 38, 48, 192):
+        for max_q in (1, 2, 15, 16, 17, 33, 96, 500, 4096, 2 ** 31 - 1):
+            need = -(-max_q // qt)
+            assert lib.tiles(1, max_q, qt) == need
+            for n in (2, 250):
+                t = lib.tiles(n, max_q, qt)
+                assert need <= t <= need + 1 and t % 2 == 1, (n, max_q, qt)
