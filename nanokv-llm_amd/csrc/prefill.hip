@@ -996,18 +996,17 @@ static int64_t split_most_tiles(int64_t n_seqs, int64_t total_q, int64_t max_seq
 // Whether the split launch is the faster one, from what the host knows of the lengths and the
 // batch's mix. In us, fitted to both sides' times of 200 random steps at head_dim 128 (1 - 104
 // sequences, 1 - 3000 new tokens, contexts of up to 16k, every KV type), what other forms change
-// to 1286 of head_dim 64 - 256 and 1 - 128 query heads a KV head:
+// and a decode row's cost to 663 of head_dim 64 - 256 and 1 - 128 query heads a KV head:
 //  * plain, the workgroup of the longest sequence's last tile walks its keys alone, 1.0 a 64-key
 //    step with the small tiles of a few workgroups; else every step of a tile costs its share
-//    of the chip, 1.5, and of a decode row 4;
+//    of the chip, 1.5, and of a decode row 2.5;
 //  * split, the tiles' steps cost the same (2.1 at head_dim 256), the rows' (their bytes) 0.25, or
 //    0.6 for each of several column groups (1 at head_dim 256), and the launch, the parts' writing
 //    and the merge 35.
-// The keys of a batch are taken as half of the longest sequence's. Of the 1286 the rule splits 548,
-// 9 of them over 10% slower than the plain launch (23% at most) and others up to 8x faster, and
-// loses 3.5% against always knowing the faster. One layer's call of 512 tokens on 12288 (Hq 32,
-// Hk 8): 181 us plain (347 with 192-row tiles), 133 split; of 48 decode rows with two 512-token
-// chunks: 237 and 123.
+// The keys of a batch are taken as half of the longest sequence's. Of the 663 the rule splits 270,
+// 3 of them over 10% slower than the plain launch (17% at most) and others up to 8x faster, and
+// loses 3.2% against always knowing the faster. 512 tokens on 12288 (Hq 32, Hk 8): 172 us plain
+// (344 with 192-row tiles), 126 split; 48 decode rows with two 512-token chunks: 202 and 118.
 static bool prefill_split_wins(int32_t n_seqs, int64_t total_q, int32_t max_seqlen_q,
                                int32_t max_seqlen_k, int32_t n_q_heads, int32_t n_kv_heads,
                                int32_t head_dim, bool f8) {
@@ -1031,7 +1030,7 @@ static bool prefill_split_wins(int32_t n_seqs, int64_t total_q, int32_t max_seql
   const int ncg = decode_ncg(g);
   const double tile_cost = head_dim == 256 ? 2.1 : 1.5;
   const double row_cost = ncg == 1 ? 0.25 : (head_dim == 256 ? 1.0 : 0.6) * ncg;
-  return dim * std::max(steps, 1.5 * tile_steps + 4.0 * row_steps) >
+  return dim * std::max(steps, 1.5 * tile_steps + 2.5 * row_steps) >
          35.0 + dim * (tile_cost * tile_steps + row_cost * row_steps);
 }
 

@@ -295,7 +295,7 @@ def test_plain_tile_sizes_match_the_oracle(nkv, dev, kind, Hq, Hk, D, n):
 # measured at 0.55 of the plain one's time or less
 SPLIT_FASTER = [(40, 135, 96, 2203, 32, 8, 256, 0), (1, 10, 10, 1748, 8, 8, 256, 2),
                 (40, 54, 15, 6000, 128, 2, 128, 2), (1, 5, 5, 3255, 48, 1, 256, 0),
-                (2, 95, 85, 11968, 28, 4, 256, 2), (40, 237, 193, 727, 8, 8, 256, 0)]
+                (2, 95, 85, 11968, 28, 4, 256, 2)]
 
 
 def test_split_plan_and_arguments_on_the_host():
