@@ -1093,7 +1093,7 @@ def main():
         "cpu_baseline": cpu,
         **comp,
         "prefill_roofline": {
-            "kernel": "prefill_varlen_kernel<false, 128, false, true>",
+            "kernel": "prefill_varlen_kernel<false, 128, false, true, 3>",
             "bound": "mfma",
             "achieved": pre["prefill_chunked_tflops"],
             "peak": MFMA_BF16_PEAK_TFLOPS,

@@ -9,17 +9,18 @@
 // any store, lanes of a wave cover consecutive chunks of one row so every
 // wave-wide load/store is a coalesced 1 KiB access, and a bounded grid strides
 // over the rest (prefill-sized token counts keep ~128 KiB in flight per CU).
-// Up to about 16k tokens (Hk 8) it is one chunk a thread, so that four times the waves share
-// them, with 32-bit index arithmetic (four 64-bit divisions a thread took longer than a decode
-// step's loads): 64 tokens 3.5 -> 2.7 us, 512 3.8 -> 2.8, 4096 6.7 -> 5.5, 9000 13.6 -> 12.9;
-// 38000 with four chunks a thread 52.3 (6.0 TB/s), with one 52.6.
+// Up to about 16k tokens (Hk 8) it is one chunk a thread at a time: four times the waves share them
+// up to 4k tokens, where the grid is full; above, the threads stride over up to four. Indexes
+// are 32 bits wide (four 64-bit divisions a thread took longer than a decode step's loads): 64
+// tokens 3.5 -> 2.7 us, 512 3.8 -> 2.8, 4096 6.7 -> 5.5, 9000 13.6 -> 12.9; 38000 with four chunks a
+// thread at once 52.3 (6.0 TB/s), with one 52.6.
 #include "nkv_common.h"
 
 namespace nkv {
 
 constexpr int kStoreThreads = 256;
 constexpr int kStoreUnroll = 4;
-constexpr int kStoreFewGroups = 16384;  // one chunk a thread up to this many workgroups of them
+constexpr int kStoreFewGroups = 16384;  // one chunk at a time up to this many workgroups' threads
 
 // Index: uint32_t where the chunks fit, else uint64_t.
 template <typename Chunk, int kUnroll, typename Index>
